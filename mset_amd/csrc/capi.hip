@@ -83,7 +83,7 @@ using ProfMap = std::map<std::string, Prof>;
 
 // scratch shared by the tilts of one reconstruction
 struct Workspace {
-    DevBuf<float2> save, trans, probeF, pslab, PG, planes;
+    DevBuf<float2> save, trans, probeF, pslab, PG, planes, lines;
     DevBuf<float> gslab, G;
     int exit_waves = MSET_EXIT_WAVES_AUTO;   // requested exit-wave variant of the batched kernels
     int slot_limit = 0;                      // cap on the persistent grid of the batched kernels (0: none)
@@ -429,46 +429,29 @@ int read_errors(mset_ctx* c, int first, int count, double* out) {
     return MSET_OK;
 }
 
-// The sequential path on the separable 256 routine: each position is a batched launch of that one position
-// (the 1024-thread shape, one workgroup) with its gradient planes, probe term and position terms, and the
-// host applies the three steps before the next position's transmission and fftn(probe).  The semantics of
-// the one-position kernel below, at one plane pass per propagation step instead of two.
-int issue_plain_sep(mset_ctx* c) {
-    Workspace& W = *c->ws;
-    CHK(W.pslab.ensure(plane(c), "probe term"));
-    CHK(c->dpos.ensure((size_t)2 * c->npos, "position terms"));
-    PosArgs A = base_args(c);
-    A.sep = 1;
-    A.waves = WAVES_STORE;
-    A.count = 1;
-    A.nslab = 1;
-    const float* s = c->p.step_size;
-    for (int k = 0; k < c->npos; ++k) {
-        HIPCHK(launch_transmission_sep(c->V.p, (float*)W.trans.p, (float*)W.trans.p + plane(c) * c->L, c->n, c->nz,
-                                       binning(c), c->p.sigma, c->p.potential_pixelsize, c->stream));
-        HIPCHK(launch_plane_fft(c->n, c->probe.p, W.probeF.p, c->tw.p, 0, 1.f, 0.f, W.planes.p, c->stream));
-        A.first = k;
-        {
-            Timed t(c, "position_plain");
-            HIPCHK(launch_batch(c->n, A, 1, 2, c->stream));
-        }
-        // the gradient planes (odd planes transposed by the routine), then the steps (STEP03_BACK.m:84-92)
-        HIPCHK(launch_untranspose_odd(W.gslab.p, c->n, c->L, c->stream));
-        if (s[0] != 0.f) HIPCHK(launch_update_volume(c->V.p, W.gslab.p, c->n, c->nz, binning(c), s[0], c->stream));
-        if (s[1] != 0.f)
-            HIPCHK(launch_plane_fft(c->n, W.pslab.p, c->probe.p, c->tw.p, 1, -s[1], 1.f, W.planes.p, c->stream));
-        if (s[2] != 0.f)
-            HIPCHK(launch_update_positions(c->x.p + k, c->y.p + k, c->dpos.p + 2 * (size_t)k, 1, s[2], c->stream));
-    }
-    return MSET_OK;
+// The sequential path as line passes over the whole device (line_passes.hip): a separable propagator, the
+// reference pairing, 64 x 64 and up.  Both ways cost about the same per plane at any depth; per position,
+// one workgroup against line passes: 137 and 71 us at 64 x 64 (6 planes), 576 and 205 us at 128 x 128 (16),
+// 4.5 ms and 0.45 ms at 256 x 256 (32).
+bool plain_lines(const mset_ctx* c) {
+    return position_lines_supported(c->n) && c->prop_sep && !sset(c) && c->p.grad_mode == GRAD_REF &&
+           !(c->ws->engine & MSET_ENGINE_GENERAL);
 }
 
 // one launch per position, sequential updates (issue only; no host synchronisation)
 int issue_plain(mset_ctx* c) {
-    CHK(ensure_fixed_buffers(c));
     CHK(c->ws->save.ensure((size_t)(c->L + 2) * plane(c), "save waves"));
+    if (plain_lines(c)) {
+        CHK(c->ws->lines.ensure(position_lines_work(c->n), "line passes"));
+        const PosArgs P = base_args(c);
+        for (int k = 0; k < c->npos; ++k) {
+            Timed t(c, "position_plain");
+            HIPCHK(launch_position_lines(c->n, P, k, c->ws->lines.p, c->stream));
+        }
+        return MSET_OK;
+    }
+    CHK(ensure_fixed_buffers(c));
     CHK(c->ws->gslab.ensure((size_t)c->L * plane(c), "gradient planes"));
-    if (sep_fwd(c) && c->p.grad_mode == GRAD_REF) return issue_plain_sep(c);
     PosArgs A = base_args(c);
     const float s1 = c->p.step_size[0];
     for (int k = 0; k < c->npos; ++k) {
@@ -731,6 +714,18 @@ int check_recon(mset_recon* r) {
         if (!r->tilts[j] || !r->tilts[j]->uploaded)
             return fail(MSET_EINVAL, "tilt " + std::to_string(j) + " has no data (call mset_recon_set_tilt)");
     return MSET_OK;
+}
+
+// A sequential pass in more launches than this is issued eagerly even when a graph is asked for: a captured
+// pass has a node per launch, and the host issues the launches faster than they run except at the smallest
+// plane of the line passes (3 tilts of 64 positions: 13.8 ms eager, 12.2 ms replayed at 64 x 64, 3.5k launches;
+// 16.6 and 16.5 ms at 128 x 128, 3.5k launches).
+constexpr size_t PLAIN_GRAPH_LAUNCHES = 65536;
+
+size_t plain_launches(const mset_recon* r) {
+    size_t n = 0;
+    for (const mset_ctx* c : r->tilts) n += (size_t)c->npos * (plain_lines(c) ? 2 * (size_t)c->L + 6 : 3);
+    return n;
 }
 
 // one update pass over every tilt (Run_MSET_recon.m:119-187), issue only
@@ -1193,7 +1188,7 @@ int mset_recon_iterate(mset_recon* r, int path, int batch, int use_graph, int po
     if (path != MSET_PATH_PLAIN && path != MSET_PATH_BATCHED) return fail(MSET_EINVAL, "bad path");
     if (path == MSET_PATH_BATCHED && batch <= 0) return fail(MSET_EINVAL, "batch must be positive");
     if (path == MSET_PATH_PLAIN) batch = 1;
-    if (use_graph && !r->profiling) {
+    if (use_graph && !r->profiling && (path != MSET_PATH_PLAIN || plain_launches(r) <= PLAIN_GRAPH_LAUNCHES)) {
         const bool same = r->exec && r->graph_key[0] == path && r->graph_key[1] == batch && r->graph_key[2] == positivity;
         if (!same) {
             drop_graph(r);

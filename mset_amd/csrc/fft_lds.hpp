@@ -142,6 +142,23 @@ template <bool INV> struct DFT<3, INV> {
     }
 };
 
+// radix-2 split into two 3-point DFTs
+template <bool INV> struct DFT<6, INV> {
+    __device__ __forceinline__ static void run(float2* v) {
+        constexpr float s3 = 0.86602540378443865f;
+        float2 e[3] = {v[0], v[2], v[4]}, o[3] = {v[1], v[3], v[5]};
+        DFT<3, INV>::run(e);
+        DFT<3, INV>::run(o);
+        o[1] = cmul(o[1], make_float2(0.5f, INV ? s3 : -s3));
+        o[2] = cmul(o[2], make_float2(-0.5f, INV ? s3 : -s3));
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            v[k] = cadd(e[k], o[k]);
+            v[k + 3] = csub(e[k], o[k]);
+        }
+    }
+};
+
 // ------------------------------------------------------------------ element points and buffer views
 // An element as the engines hand it to functors: its coordinates and its index in the layout the
 // current orientation streams (row-major [y][x] when consecutive lanes run along x, transposed [x][y]

@@ -79,9 +79,35 @@ __host__ __device__ inline int checkpoint_segment(int L) {
 }
 __host__ __device__ inline int checkpoint_planes(int L, int K) { return L / K + K + 3; }
 
+// Arguments of one line pass of the sequential path (line_passes.hip)
+struct LineArgs {
+    const float2* in;            // the wave, lines contiguous
+    float2* out;                 // the wave, transposed
+    const float2* tw;            // W_N^k, k < N
+    const float2* p1d;           // propagator factors px[N], py[N]
+    float2* phi;                 // sub-pixel shift factors along x [N], along y [N]
+    float* V;                    // volume [z][y][x]
+    float2* wave;                // psi of the pass's plane, lines contiguous (written forward, read back)
+    const float2* psi0;          // incident wave [y][x]
+    float2* probe;               // [y][x]
+    const float* sqrtM;          // the position's pattern, [x][y]
+    float *x, *y;                // the position
+    double* err;                 // its loss
+    double* part;                // per-workgroup sums: loss, position terms
+    int a, nz, bin;              // plane, volume depth, slices per plane
+    int head;                    // ADJ: the first adjoint pass, whose input lacks the half-step
+    int want_pos;
+    float sigma, dx, cent, s1, s2, s3;
+};
+
 bool plane_size_supported(int n);
 int position_threads(int n);
 hipError_t launch_plain(int n, const PosArgs& A, int k, hipStream_t st);
+// sequential path as line passes over the device (separable propagator, reference pairing): position k of P
+// with V, the probe and the position updated; work: position_lines_work(n) elements
+bool position_lines_supported(int n);
+size_t position_lines_work(int n);
+hipError_t launch_position_lines(int n, const PosArgs& P, int k, float2* work, hipStream_t st);
 // shape: the workgroup shape of the batched kernel (0, or 1 = the alternative shape, stored waves only)
 // shape: 0 default, 1 alternative (MSET_ENGINE_ALT_SHAPE, stored waves), 2 the separable 256 routine's
 // 1024-thread shape for launches of at most one position per CU (stored or checkpointed waves)

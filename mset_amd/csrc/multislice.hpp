@@ -10,8 +10,8 @@
 // element-wise steps ride on the FFT stages' loads and stores (fft_lds.hpp).
 //
 // Three kinds of launch share it:
-//   K_PLAIN  one position per launch, sequential semantics of src/Run_MSET_recon.m:134-158 and
-//            src/CUDA/mset.cu:107-333: the transmission planes are recomputed from V at the start, and
+//   K_PLAIN  one position per launch (where line_passes.hip does not apply), sequential semantics of
+//            src/Run_MSET_recon.m:134-158 and src/CUDA/mset.cu:107-333: the transmission planes are recomputed from V at the start, and
 //            V, the probe and the position are updated in place at the end, before the next launch.
 //   K_BATCH  many positions per launch at a fixed (V, probe): a persistent grid of workgroups, each
 //            accumulating its positions' object gradient into a private slab (L planes) and its
@@ -539,8 +539,8 @@ __device__ __forceinline__ void process_position(const PosArgs& A, int k, int sl
 // its wave: the forward sweep's own arithmetic, about one forward sweep more in all.
 //
 // Used for the batched gradient with the reference pairing and stored or checkpointed waves, and for the
-// forward-only kernels; the sequential kernel, the exact pairing and the recomputed waves use
-// process_position.
+// forward-only kernels; the exact pairing and the recomputed waves use process_position, the sequential path
+// line_passes.hip.
 template <int N, int NT, int KIND, int WV = WAVES_STORE, class Eng>
 __device__ __forceinline__ void process_sep(const PosArgs& A, int k, int slot, int slab, bool first, Eng& E,
                                             float2* phx, float2* phy, const float2* px, const float2* py,
