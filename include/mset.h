@@ -155,8 +155,8 @@ int mset_set_slot_limit(mset_ctx* ctx, int slots);
  * does, checked at upload), the forward kernels and the reference-pairing batched gradient with stored
  * waves run the separable routine, which applies the two 1D half-steps of neighbouring planes in one pass
  * over the plane (half the passes).  GENERAL: always the 2D routine.  ALT_SHAPE: the batched kernel with
- * stored waves runs the alternative workgroup shape of its plane size: twice the threads per position of
- * the LDS engine up to 64, 1024 threads at 96, at 128 the register engine with a half-size transpose
+ * stored waves runs the alternative workgroup shape of its plane size: fewer threads per position of the LDS
+ * engine at 24, 32, 64 and 96 (more at 16 and 48), at 128 the register engine with a half-size transpose
  * buffer and a 128-register budget (two workgroups per CU instead of one), at 256 16-line tiles with 256
  * threads (three workgroups per CU instead of two).  The flags combine. */
 #define MSET_ENGINE_AUTO 0

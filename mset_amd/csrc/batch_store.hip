@@ -8,9 +8,10 @@ namespace mset {
 hipError_t launch_batch_variant(int n, const PosArgs& A, int grid, int shape, hipStream_t st);
 
 hipError_t launch_batch(int n, const PosArgs& A, int grid, int shape, hipStream_t st) {
-    // shape 1: stored waves; shape 2 (1024 threads): the separable 256 routine, stored or checkpointed waves
+    // shape 1: stored waves; shape 2: stored waves at 48, or the separable 256 routine with stored or
+    // checkpointed waves
     if (shape == 1 && A.waves != WAVES_STORE) return hipErrorInvalidValue;
-    if (shape == 2 && (n != 256 || !A.sep)) return hipErrorInvalidValue;
+    if (shape == 2 && !(n == 256 && A.sep) && !(n == 48 && A.waves == WAVES_STORE)) return hipErrorInvalidValue;
     if (shape < 0 || shape > 2) return hipErrorInvalidValue;
     if (A.waves != WAVES_STORE) return launch_batch_variant(n, A, grid, shape, st);
     if (A.sep) {
@@ -18,6 +19,11 @@ hipError_t launch_batch(int n, const PosArgs& A, int grid, int shape, hipStream_
         if (shape == 2) hipLaunchKernelGGL((k_batch<256, 2, WAVES_STORE, true>), dim3(grid), dim3(Cfg<256, 2>::NT), 0, st, A);
         else if (shape) hipLaunchKernelGGL((k_batch<256, 1, WAVES_STORE, true>), dim3(grid), dim3(Cfg<256, 1>::NT), 0, st, A);
         else hipLaunchKernelGGL((k_batch<256, 0, WAVES_STORE, true>), dim3(grid), dim3(Cfg<256>::NT), 0, st, A);
+    } else if (shape == 2) {
+        if (A.pfac && !A.sset) hipLaunchKernelGGL((k_batch<48, 2, WAVES_STORE, false, true>), dim3(grid), dim3(Cfg<48, 2>::NT), 0, st, A);
+        else hipLaunchKernelGGL((k_batch<48, 2, WAVES_STORE, false>), dim3(grid), dim3(Cfg<48, 2>::NT), 0, st, A);
+    } else if (shape && A.pfac && n < 128 && !A.sset) {
+        MSET_DISPATCH_SMALL(n, hipLaunchKernelGGL((k_batch<NN, 1, WAVES_STORE, false, true>), dim3(grid), dim3(Cfg<NN, 1>::NT), 0, st, A))
     } else if (shape) {
         MSET_DISPATCH(n, hipLaunchKernelGGL((k_batch<NN, 1, WAVES_STORE, false>), dim3(grid), dim3(Cfg<NN, 1>::NT), 0, st, A))
     } else if (A.pfac && n != 256 && !A.sset) {

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <array>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -284,9 +285,11 @@ bool sep_batch(const mset_ctx* c) {
     return sep_fwd(c) && c->p.grad_mode == GRAD_REF && (c->ws->waves == WAVES_STORE || c->ws->waves == WAVES_CHECKPOINT);
 }
 
-// workgroup shape of a batched call: the alternative shape (MSET_ENGINE_ALT_SHAPE) exists for stored waves
-int shape_for(const mset_ctx* c, int waves) {
-    return (c->ws->engine & MSET_ENGINE_ALT_SHAPE) && waves == WAVES_STORE ? 1 : 0;
+// workgroup shape of a batched call: the alternative shape (MSET_ENGINE_ALT_SHAPE) exists for stored waves; a
+// gradient request (fixed) takes it below 128 as well, see Cfg
+int shape_for(const mset_ctx* c, int waves, bool fixed) {
+    const bool alt = (c->ws->engine & MSET_ENGINE_ALT_SHAPE) || (fixed && c->n < 128 && c->n != 48);
+    return alt && waves == WAVES_STORE ? 1 : 0;
 }
 
 // workgroups of the batched kernel of a workgroup shape the device keeps resident at once (1 per CU at
@@ -314,18 +317,23 @@ int batch_slots(mset_ctx* c) { return batch_slots(c, c->ws->shape); }
 int grad_slabs(mset_ctx* c, int shape) { return std::max(1, std::min(device_slots(c, shape), c->npos)); }
 int grad_slabs(mset_ctx* c) { return grad_slabs(c, c->ws->shape); }
 
+// The workgroup shape of a batched launch.  A launch with at most one position per CU takes the large workgroup
+// where the default one is sized for several positions per CU: with stored waves at 48 (201 -> 128 us at 256
+// positions x 12 planes; from 400 on the default is faster, 220 against 248), and in the separable 256 routine
+// with stored or checkpointed waves (a tilt's last mini-batch, 15-20 % shorter at 64-256 positions).  The line
+// transforms, operand order and slab assignment are the default shape's, so the gradient slabs are the same up
+// to the compiler's contraction of products (bit for bit at 256); the workgroup sums (loss, position terms)
+// add their terms in another order.
+int batch_shape(const mset_ctx* c, int shape, bool sep, int waves, int count, bool fixed) {
+    if (shape != 0 || count > c->cus) return shape;
+    if (c->n == 48 && waves == WAVES_STORE && !fixed) return 2;
+    return c->n == 256 && sep && (waves == WAVES_STORE || waves == WAVES_CHECKPOINT) ? 2 : 0;
+}
+// the same for the forward-only kernels (78 -> 62 us at 48 and up to 256 positions, 94 against 117 at 400)
+int fwd_shape(const mset_ctx* c, int count) { return c->n == 48 && count <= c->cus ? 2 : 0; }
+
 // grid of a batched launch of `count` positions on S slabs: at most `want` workgroups and, when slabs take
 // several positions (count > S), a divisor of S, so that each slab's positions run on one workgroup in order
-// The workgroup shape of a batched launch: a launch of the separable 256 routine (stored or checkpointed
-// waves) with at most one position per CU (a tilt's last mini-batch) runs the 1024-thread shape, one
-// workgroup of 16 waves per CU instead of one or two of 8 (15-20 % shorter at 64-256 positions).  Its line
-// transforms, operand order and slab assignment are the default shape's, so the gradient slabs are the
-// same bit for bit; only the workgroup sums (loss, position terms) add their terms in another order.
-int batch_shape(const mset_ctx* c, int shape, bool sep, int waves, int count) {
-    const bool wide = waves == WAVES_STORE || waves == WAVES_CHECKPOINT;
-    return c->n == 256 && shape == 0 && sep && wide && count <= c->cus ? 2 : shape;
-}
-
 int launch_grid(int want, int count, int S) {
     int g = std::max(1, std::min(want, count));
     if (count > S)
@@ -380,12 +388,12 @@ int resolve_exit_waves(mset_ctx* c, int slots, int* waves) {
     return MSET_OK;
 }
 
-int ensure_batch_buffers(mset_ctx* c) {
+int ensure_batch_buffers(mset_ctx* c, bool fixed) {
     Workspace& W = *c->ws;
     int wv = WAVES_STORE;
     CHK(resolve_exit_waves(c, batch_slots(c, 0), &wv));
     W.waves = wv;
-    W.shape = shape_for(c, wv);
+    W.shape = shape_for(c, wv, fixed);
     const int s = batch_slots(c);
     CHK(ensure_fixed_buffers(c));
     const int save_planes = wave_planes(c, wv);
@@ -477,7 +485,7 @@ int issue_fwd(mset_ctx* c, float* inten) {
     A.count = c->npos;
     A.inten = inten;
     Timed t(c, "position_fwd");
-    HIPCHK(launch_fwd(c->n, A, batch_slots(c), c->stream));
+    HIPCHK(launch_fwd(c->n, A, plane_in_global(c->n) ? batch_slots(c) : batch_slots(c, 0), fwd_shape(c, c->npos), c->stream));
     return MSET_OK;
 }
 
@@ -485,7 +493,7 @@ int issue_fwd(mset_ctx* c, float* inten) {
 // direction, real space) and c->dpos; with apply, the steps are taken (RVol += s1 G, probe -= s2 PG,
 // positions += s3 dpos).  want: the terms to form (the gradient request forms all of them).
 int issue_grad(mset_ctx* c, int first, int count, bool apply, int want) {
-    CHK(ensure_batch_buffers(c));
+    CHK(ensure_batch_buffers(c, !apply));
     const bool sep = sep_batch(c);
     CHK(prepare_fixed(c, sep ? 2 : 0));
     Workspace& W = *c->ws;
@@ -501,7 +509,7 @@ int issue_grad(mset_ctx* c, int first, int count, bool apply, int want) {
     // every used slab receives at least one position, and its first one writes it
     {
         Timed t(c, "position_batch");
-        HIPCHK(launch_batch(c->n, A, grid, batch_shape(c, W.shape, sep, W.waves, count), c->stream));
+        HIPCHK(launch_batch(c->n, A, grid, batch_shape(c, W.shape, sep, W.waves, count, !apply), c->stream));
     }
     HIPCHK(launch_reduce_slabs(W.gslab.p, used, (size_t)planes(c) * plane(c), W.G.p, c->stream));
     if (sep) HIPCHK(launch_untranspose_odd(W.G.p, c->n, c->L, c->stream));
@@ -882,7 +890,7 @@ int mset_grad_noalloc(mset_ctx* c, int first, int count, float* dV, float* dprob
     auto need = [&](int S, int G) { return fixed + (size_t)S * (s_g + s_ps) + (size_t)G * (s_save + s_pl); };
     // mset_grad's slabs and grid when they fit (then the sums are bitwise mset_grad's), else as many resident
     // positions as fit, one slab each
-    const int shape = shape_for(c, WAVES_STORE);
+    const int shape = shape_for(c, WAVES_STORE, true);
     int S = std::min(grad_slabs(c, shape), count);
     int G = launch_grid(batch_slots(c, shape), count, S);
     while (G > 1 && need(S, G) > MSET_NOALLOC_SCRATCH_BYTES) G = launch_grid(G - 1, count, S);
@@ -926,7 +934,7 @@ int mset_grad_noalloc(mset_ctx* c, int first, int count, float* dV, float* dprob
     A.sep = sep ? 1 : 0;
     A.tph = (const float*)trans;
     A.tph_b = (const float*)trans + L * n2;
-    HIPCHK(launch_batch(c->n, A, G, batch_shape(c, shape, sep, WAVES_STORE, count), c->stream));
+    HIPCHK(launch_batch(c->n, A, G, batch_shape(c, shape, sep, WAVES_STORE, count, true), c->stream));
     HIPCHK(launch_reduce_slabs(gslab, S, L * n2, dV, c->stream));
     if (sep) HIPCHK(launch_untranspose_odd(dV, c->n, c->L, c->stream));
     HIPCHK(launch_reduce_cslabs(pslab, S, n2, pslab, c->stream));
@@ -938,7 +946,7 @@ int mset_waves(mset_ctx* c, int k, float* waves_out) {
     CHK(check_uploaded(c));
     if (k < 0 || k >= c->npos || !waves_out) return fail(MSET_EINVAL, "bad position index or null output");
     CHK(set_method(c, MSET_METHOD_MSET));
-    CHK(ensure_batch_buffers(c));
+    CHK(ensure_batch_buffers(c, true));
     CHK(prepare_fixed(c));
     // every plane's wave is read back: the store layout, in slot 0
     CHK(c->ws->save.ensure((size_t)(c->L + 2) * plane(c), "save waves"));
@@ -948,7 +956,7 @@ int mset_waves(mset_ctx* c, int k, float* waves_out) {
     A.want = 0;
     A.waves = WAVES_STORE;
     A.nslab = 1;
-    HIPCHK(launch_batch(c->n, A, 1, 0, c->stream));
+    HIPCHK(launch_batch(c->n, A, 1, c->n < 128 && c->n != 48 ? 1 : 0, c->stream));
     HIPCHK(hipMemcpyAsync(waves_out, c->ws->save.p, sizeof(float2) * (size_t)(c->L + 1) * plane(c),
                           hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1290,7 +1298,7 @@ int mset_recon_error_pass(mset_recon* r, double* errs) {
     A.sep = sep ? 1 : 0;
     {
         Timed t(c0, "position_fwd");
-        HIPCHK(launch_fwd_tilts(r->n, A, grid, r->stream));
+        HIPCHK(launch_fwd_tilts(r->n, A, grid, fwd_shape(c0, (int)std::min<size_t>(tot, INT_MAX)), r->stream));
     }
     std::vector<double> e(tot);
     HIPCHK(hipMemcpyAsync(e.data(), r->err_all.p, sizeof(double) * tot, hipMemcpyDeviceToHost, r->stream));

@@ -108,13 +108,13 @@ hipError_t launch_plain(int n, const PosArgs& A, int k, hipStream_t st);
 bool position_lines_supported(int n);
 size_t position_lines_work(int n);
 hipError_t launch_position_lines(int n, const PosArgs& P, int k, float2* work, hipStream_t st);
-// shape: the workgroup shape of the batched kernel (0, or 1 = the alternative shape, stored waves only)
-// shape: 0 default, 1 alternative (MSET_ENGINE_ALT_SHAPE, stored waves), 2 the separable 256 routine's
-// 1024-thread shape for launches of at most one position per CU (stored or checkpointed waves)
+// shape: 0 default, 1 alternative (MSET_ENGINE_ALT_SHAPE, stored waves), 2 the large workgroup for launches of
+// at most one position per CU (at 48 with stored waves; the separable 256 routine, stored or checkpointed)
 hipError_t launch_batch(int n, const PosArgs& A, int grid, int shape, hipStream_t st);
-hipError_t launch_fwd(int n, const PosArgs& A, int grid, hipStream_t st);
+// shape: 0, or 2 at 48 as above
+hipError_t launch_fwd(int n, const PosArgs& A, int grid, int shape, hipStream_t st);
 // forward + loss over the work items A.order[0 .. A.count) of several tilts (A.tilts)
-hipError_t launch_fwd_tilts(int n, const PosArgs& A, int grid, hipStream_t st);
+hipError_t launch_fwd_tilts(int n, const PosArgs& A, int grid, int shape, hipStream_t st);
 // 2D transform of one plane: dir 0 forward, in [y][x] -> out [x][y]; dir 1 inverse, in [x][y] -> out [y][x]
 // = alpha/N^2 v + beta out, and with out2 also out2 = alpha2/N^2 v + beta2 out2.  planes: at N = 256 one
 // plane of scratch (the transform runs as two passes of line transforms over the device).

@@ -24,13 +24,14 @@ int position_threads(int n) {
 }
 
 hipError_t launch_plain(int n, const PosArgs& A, int k, hipStream_t st) {
-    if (A.pfac && n != 256 && !A.sset)
-        MSET_DISPATCH_SMALL(n, hipLaunchKernelGGL((k_plain<NN, true>), dim3(1), dim3(Cfg<NN>::NT), 0, st, A, k))
+    // one position: the shape of launches that leave CUs idle (at 256 the general routine has the default one)
+    if (n == 256) hipLaunchKernelGGL((k_plain<256, 0>), dim3(1), dim3(Cfg<256>::NT), 0, st, A, k);
+    else if (A.pfac && !A.sset)
+        MSET_DISPATCH_SMALL(n, hipLaunchKernelGGL((k_plain<NN, 2, true>), dim3(1), dim3(Cfg<NN, 2>::NT), 0, st, A, k))
     else
-        MSET_DISPATCH(n, hipLaunchKernelGGL((k_plain<NN, false>), dim3(1), dim3(Cfg<NN>::NT), 0, st, A, k));
+        MSET_DISPATCH_SMALL(n, hipLaunchKernelGGL((k_plain<NN, 2>), dim3(1), dim3(Cfg<NN, 2>::NT), 0, st, A, k))
     return hipGetLastError();
 }
-
 
 hipError_t launch_plane_fft(int n, const float2* in, float2* out, const float2* tw, int dir, float alpha, float beta,
                             float2* planes, hipStream_t st, float2* out2, float alpha2, float beta2) {

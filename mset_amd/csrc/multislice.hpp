@@ -38,32 +38,47 @@
 
 namespace mset {
 
-// plane engine and workgroup size per plane size: register-resident at 128, LDS stages elsewhere
 // Engine and workgroup shape per plane size.  NT threads; MINB: waves per SIMD the register budget must allow
-// (HIP launch bounds).  SH = 0: the shape every kernel uses; SH = 1: the alternative shape of the batched
-// kernel, a candidate for the autotuner (MSET_ENGINE_ALT_SHAPE): twice the threads per position of the LDS
-// engine up to N = 64, 1024 threads at 96, at 128 the register engine with a half-size transpose buffer and a
-// 128-register budget (two workgroups per CU instead of one; it spills about 400 registers), and tiles of 16
-// lines with 256 threads (three workgroups per CU instead of two) at 256.
+// (HIP launch bounds).
+//
+// SH = 0: the shape of the batched and forward-only kernels.  Below 128 a position's time is the latency of its
+// chain of short LDS stages, so it takes enough threads for 4 to 12 elements each with the staged operands
+// loaded together ahead of the stage (AHEAD), rather than 9 to 18 elements with one load latency each.
+// Batched gradient of 256 / 1400 positions x 12 planes, 64 to 256 threads (576 at 96) against the shapes here:
+// 51 -> 44 / 68 -> 54 us at 16, 120 -> 70 / 157 -> 160 at 24, 211 -> 73 / 256 -> 170 at 32,
+// 301 -> 169 / 920 -> 780 at 64, and 726 -> 415 us for 256, 2108 -> 1229 for 700 positions at 96.  (At 64 a
+// budget of 4 waves per SIMD, two workgroups per CU, is 7 % slower at 256 positions and 14 % faster at 1400.)
+// At 48 the small workgroup is the better one once positions share a CU (654 against 721 us at 1400) and
+// the large one, SH = 2, below that (201 -> 128 us at 256).
+// SH = 1: the alternative shape of the batched kernel, a candidate for the autotuner (MSET_ENGINE_ALT_SHAPE):
+// smaller workgroups with operands loaded element by element (at 48 a larger one); at 128 the register engine
+// with a half-size transpose buffer and a 128-register budget (two workgroups per CU instead of one; it spills
+// about 400 registers); tiles of 16 lines with 256 threads (three workgroups per CU instead of two) at 256.
+// Below 128 (other than 48) mset_grad runs this shape: the compiler contracts the products of the two differently
+// (2e-7 of the waves), which position terms that cancel turn into 1e-4 of a gradient, and gradients are
+// what callers difference.
+// SH = 2: launches of at most one position per CU and the one-position kernel: at 48 a workgroup of 768, at 256
+// 64-line tiles, one workgroup of 16 waves per CU with twice the default workgroup's loads in flight; the
+// default shape elsewhere.
 template <int N, int SH = 0> struct Cfg;
-template <> struct Cfg<16> { static constexpr int NT = 64, MINB = 1;  using Eng = LdsEngine<16, 64>; };
-template <> struct Cfg<24> { static constexpr int NT = 64, MINB = 1;  using Eng = LdsEngine<24, 64>; };
-template <> struct Cfg<32> { static constexpr int NT = 64, MINB = 1;  using Eng = LdsEngine<32, 64>; };
+template <> struct Cfg<16> { static constexpr int NT = 64, MINB = 1;  using Eng = LdsEngine<16, 64, true>; };
+template <> struct Cfg<24> { static constexpr int NT = 192, MINB = 1; using Eng = LdsEngine<24, 192, true>; };
+template <> struct Cfg<32> { static constexpr int NT = 256, MINB = 1; using Eng = LdsEngine<32, 256, true>; };
 template <> struct Cfg<48> { static constexpr int NT = 192, MINB = 1; using Eng = LdsEngine<48, 192>; };
-template <> struct Cfg<64> { static constexpr int NT = 256, MINB = 3; using Eng = LdsEngine<64, 256>; };
-template <> struct Cfg<96> { static constexpr int NT = 576, MINB = 1; using Eng = LdsEngine<96, 576>; };
+template <> struct Cfg<64> { static constexpr int NT = 512, MINB = 4; using Eng = LdsEngine<64, 512, true>; };
+template <> struct Cfg<96> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<96, 768, true>; };
 template <> struct Cfg<128> { static constexpr int NT = 512, MINB = 1; using Eng = RegEngine<128>; };
 template <> struct Cfg<256> { static constexpr int NT = 512, MINB = 4; using Eng = TiledEngine<256, 512>; };
-template <> struct Cfg<16, 1> { static constexpr int NT = 128, MINB = 1; using Eng = LdsEngine<16, 128>; };
-template <> struct Cfg<24, 1> { static constexpr int NT = 128, MINB = 1; using Eng = LdsEngine<24, 128>; };
-template <> struct Cfg<32, 1> { static constexpr int NT = 128, MINB = 1; using Eng = LdsEngine<32, 128>; };
+template <> struct Cfg<16, 1> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<16, 64>; };
+template <> struct Cfg<24, 1> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<24, 64>; };
+template <> struct Cfg<32, 1> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<32, 64>; };
 template <> struct Cfg<48, 1> { static constexpr int NT = 384, MINB = 1; using Eng = LdsEngine<48, 384>; };
-template <> struct Cfg<64, 1> { static constexpr int NT = 512, MINB = 1; using Eng = LdsEngine<64, 512>; };
-template <> struct Cfg<96, 1> { static constexpr int NT = 1024, MINB = 1; using Eng = LdsEngine<96, 1024>; };
+template <> struct Cfg<64, 1> { static constexpr int NT = 256, MINB = 3; using Eng = LdsEngine<64, 256>; };
+template <> struct Cfg<96, 1> { static constexpr int NT = 576, MINB = 1; using Eng = LdsEngine<96, 576>; };
 template <> struct Cfg<128, 1> { static constexpr int NT = 512, MINB = 4; using Eng = RegEngine<128, true>; };
 template <> struct Cfg<256, 1> { static constexpr int NT = 256, MINB = 3; using Eng = TiledEngine<256, 256>; };
-// launches of at most one position per CU (a tilt's last mini-batch): 64-line tiles, one workgroup of 16 waves
-// per CU, twice the default workgroup's loads in flight
+template <int N> struct Cfg<N, 2> : Cfg<N> {};
+template <> struct Cfg<48, 2> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<48, 768, true>; };
 template <> struct Cfg<256, 2> { static constexpr int NT = 1024, MINB = 4; using Eng = TiledEngine<256, 1024>; };
 
 
@@ -826,10 +841,10 @@ template <int N, int NT> __device__ __forceinline__ void load_twiddles(float2* t
     E.init(s, tw);
 
 // PFAC: the propagator as its 1D factors from LDS (a separable propagator), as in the batched kernel
-template <int N, bool PFAC = false>
-__global__ __launch_bounds__(Cfg<N>::NT, Cfg<N>::MINB) void k_plain(PosArgs A, int k) {
-    constexpr int NT = Cfg<N>::NT;
-    MSET_LDS(N, NT, 0)
+template <int N, int SH, bool PFAC = false>
+__global__ __launch_bounds__((Cfg<N, SH>::NT), (Cfg<N, SH>::MINB)) void k_plain(PosArgs A, int k) {
+    constexpr int NT = Cfg<N, SH>::NT;
+    MSET_LDS(N, NT, SH)
     float2* pxs = nullptr;
     float2* pys = nullptr;
     if constexpr (PFAC) {
@@ -883,10 +898,10 @@ __global__ __launch_bounds__((Cfg<N, SH>::NT), (Cfg<N, SH>::MINB)) void k_batch(
 // MT: the work items are positions of several tilts (A.tilts, A.order), so a whole error pass over a tilt
 // series is one persistent launch; a separate instantiation, so the one-tilt kernel carries none of it
 // PFAC (general routine below 256): the propagator as its 1D factors from LDS.
-template <int N, bool MT, bool SEP, bool PFAC = false>
-__global__ __launch_bounds__(Cfg<N>::NT, Cfg<N>::MINB) void k_fwd(PosArgs A) {
-    constexpr int NT = Cfg<N>::NT;
-    MSET_LDS(N, NT, 0)
+template <int N, int SH, bool MT, bool SEP, bool PFAC = false>
+__global__ __launch_bounds__((Cfg<N, SH>::NT), (Cfg<N, SH>::MINB)) void k_fwd(PosArgs A) {
+    constexpr int NT = Cfg<N, SH>::NT;
+    MSET_LDS(N, NT, SH)
     float2* px = nullptr;
     float2* py = nullptr;
     if constexpr (SEP || PFAC) {
