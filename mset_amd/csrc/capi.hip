@@ -667,14 +667,19 @@ int upload_impl(mset_ctx* c, const mset_params* p, const float* RVol, const floa
     return MSET_OK;
 }
 
-int rotate_volume(mset_ctx* c, float* vol, const double* v1, const double* v2, const double* v3, const double* ang,
-                  bool inverse) {
+// vol = rotation of src (src may be vol)
+int rotate_volume(mset_ctx* c, const float* src, float* vol, const double* v1, const double* v2, const double* v3,
+                  const double* ang, bool inverse) {
     double R[9];
-    if (!rot_matrix(v1, v2, v3, ang[0], ang[1], ang[2], inverse, R)) return MSET_OK;   // |angles| <= 0.5
+    if (!rot_matrix(v1, v2, v3, ang[0], ang[1], ang[2], inverse, R)) {   // |angles| <= 0.5
+        if (src != vol)
+            HIPCHK(hipMemcpyAsync(vol, src, sizeof(float) * plane(c) * c->nz, hipMemcpyDeviceToDevice, c->stream));
+        return MSET_OK;
+    }
     if (!rot_size_supported(c->n) || !rot_size_supported(c->nz))
         return fail(MSET_EUNSUPPORTED, "rotation line length not built");
     Timed t(c, "rotate");
-    const int r = rot_run(c->ws->rot, vol, c->n, c->n, c->nz, R, 11.0, c->stream);
+    const int r = rot_run(c->ws->rot, src, vol, c->n, c->n, c->nz, R, 11.0, c->stream);
     if (r != MSET_OK) return fail(r, rot_last_error());
     return MSET_OK;
 }
@@ -742,14 +747,12 @@ int issue_update_pass(mset_recon* r, int path, int batch, int positivity) {
     for (size_t j = 0; j < r->tilts.size(); ++j) {
         mset_ctx* c = r->tilts[j];
         // STEP01: RVol = inv_rot(rec)
-        HIPCHK(hipMemcpyAsync(c->V.p, r->rec.p, sizeof(float) * nv, hipMemcpyDeviceToDevice, r->stream));
-        CHK(rotate_volume(c, c->V.p, r->vec, r->vec + 3, r->vec + 6, r->angles[j].data(), true));
+        CHK(rotate_volume(c, r->rec.p, c->V.p, r->vec, r->vec + 3, r->vec + 6, r->angles[j].data(), true));
         // STEP02-04
         if (path == MSET_PATH_PLAIN) CHK(issue_plain(c));
         else CHK(issue_batched(c, batch));
         // STEP05: rec = rot(RVol), positivity
-        HIPCHK(hipMemcpyAsync(r->rec.p, c->V.p, sizeof(float) * nv, hipMemcpyDeviceToDevice, r->stream));
-        CHK(rotate_volume(c, r->rec.p, r->vec, r->vec + 3, r->vec + 6, r->angles[j].data(), false));
+        CHK(rotate_volume(c, c->V.p, r->rec.p, r->vec, r->vec + 3, r->vec + 6, r->angles[j].data(), false));
         if (positivity) HIPCHK(launch_positivity(r->rec.p, nv, r->stream));
     }
     return MSET_OK;
@@ -1023,7 +1026,7 @@ int mset_rotate(mset_ctx* c, const float* in, float* out, int nx, int ny, int nz
     HIPCHK(hipMemcpyAsync(buf.p, in, sizeof(float) * nv, hipMemcpyHostToDevice, c->stream));
     {
         Timed t(c, "rotate");
-        const int r = rot_run(c->ws->rot, buf.p, nx, ny, nz, R, step, c->stream);
+        const int r = rot_run(c->ws->rot, buf.p, buf.p, nx, ny, nz, R, step, c->stream);
         if (r != MSET_OK) return fail(r, rot_last_error());
     }
     HIPCHK(hipMemcpyAsync(out, buf.p, sizeof(float) * nv, hipMemcpyDeviceToHost, c->stream));
@@ -1096,7 +1099,7 @@ int mset_rotate_resident(mset_ctx* c, const double* v1, const double* v2, const 
     CHK(check_uploaded(c));
     if (!v1 || !v2 || !v3) return fail(MSET_EINVAL, "null rotation axis");
     const double ang[3] = {phi, theta, psi};
-    CHK(rotate_volume(c, c->V.p, v1, v2, v3, ang, inverse != 0));
+    CHK(rotate_volume(c, c->V.p, c->V.p, v1, v2, v3, ang, inverse != 0));
     HIPCHK(hipStreamSynchronize(c->stream));
     return MSET_OK;
 }
@@ -1272,8 +1275,7 @@ int mset_recon_error_pass(mset_recon* r, double* errs) {
     for (int j = 0; j < T; ++j) {
         mset_ctx* c = r->tilts[j];
         CHK(set_method(c, MSET_METHOD_MSET));
-        HIPCHK(hipMemcpyAsync(c->V.p, r->rec.p, sizeof(float) * nv, hipMemcpyDeviceToDevice, r->stream));
-        CHK(rotate_volume(c, c->V.p, r->vec, r->vec + 3, r->vec + 6, r->angles[j].data(), true));
+        CHK(rotate_volume(c, r->rec.p, c->V.p, r->vec, r->vec + 3, r->vec + 6, r->angles[j].data(), true));
         CHK(c->mt_trans.ensure((size_t)c->L * plane(c), "tilt transmission"));
         CHK(c->mt_probeF.ensure(plane(c), "tilt probe spectrum"));
         if (sep)

@@ -38,94 +38,14 @@
 // 5 to 6 us at 128, about 2 of them the launch and the loads.
 #include <hip/hip_runtime.h>
 
-#include "fft_lds.hpp"
 #include "kernels.hpp"
+#include "line_fft.hpp"
 
 namespace mset {
 
 namespace {
 
-// radices of a line transform: the first and the last are 4, so a thread's points j + r N / 4 are both the
-// input of the first stage and the output of the last and stay in registers between transforms
-template <int N> struct LinePlan;
-template <> struct LinePlan<64>  { static constexpr int S = 3; static constexpr int R[4] = {4, 4, 4, 1}; };
-template <> struct LinePlan<96>  { static constexpr int S = 3; static constexpr int R[4] = {4, 6, 4, 1}; };
-template <> struct LinePlan<128> { static constexpr int S = 3; static constexpr int R[4] = {4, 8, 4, 1}; };
-template <> struct LinePlan<256> { static constexpr int S = 4; static constexpr int R[4] = {4, 4, 4, 4}; };
-
 constexpr int TL = 4;      // lines per workgroup
-constexpr int E = 4;       // points per thread
-// LDS slot of a point of a line: 4 lines side by side, one pad group after every 4 points.  8 lanes of
-// consecutive j (one pass of 64-bit accesses over the banks) then fall on 8 different 32-byte groups for
-// the stage-1 and stage-2 writes, and on at most two shared ones otherwise.
-__device__ __forceinline__ int slot(int pos, int line) { return (pos + (pos >> 2)) * TL + line; }
-template <int N> constexpr int lds_half() { return (N + N / 4) * TL; }
-
-template <int N> struct Line {
-    using P = LinePlan<N>;
-    static constexpr int T = N / E;            // threads per line
-    static constexpr int RM = P::R[1];         // radix of the second stage (and, at 256, of the third)
-    float2* s;                                 // two exchange buffers
-    int buf, line, j;
-    float2 w1[RM - 1], w2[3], w3[3];           // twiddles of the second, (third) and last stage
-
-    __device__ __forceinline__ void init(float2* lds, const float2* __restrict__ tw) {
-        s = lds;
-        buf = 0;
-        line = threadIdx.x % TL;
-        j = threadIdx.x / TL;
-        constexpr int NL = N / (4 * RM);       // table stride of the second stage
-        const int k1 = j % 4;
-#pragma unroll
-        for (int r = 1; r < RM; ++r) w1[r - 1] = tw[k1 * r * NL];
-        if constexpr (P::S == 4) {
-            const int k2 = j % 16;
-#pragma unroll
-            for (int r = 1; r < 4; ++r) w2[r - 1] = tw[k2 * r * (N / 64)];
-        }
-#pragma unroll
-        for (int r = 1; r < 4; ++r) w3[r - 1] = tw[j * r];
-    }
-
-    template <int R, int NS, bool INV, int NW>
-    __device__ __forceinline__ void mid(const float2 (&w)[NW]) {
-        float2* a = s + buf;
-        buf = lds_half<N>() - buf;
-        float2* b = s + buf;
-        constexpr int NB = N / R;
-        if (T == NB || j < NB) {
-            float2 u[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) u[r] = a[slot(j + r * NB, line)];
-#pragma unroll
-            for (int r = 1; r < R; ++r) u[r] = INV ? cmulc(u[r], w[r - 1]) : cmul(u[r], w[r - 1]);
-            DFT<R, INV>::run(u);
-            const int base = (j / NS) * NS * R + j % NS;
-#pragma unroll
-            for (int r = 0; r < R; ++r) b[slot(base + r * NS, line)] = u[r];
-        }
-        __syncthreads();
-    }
-
-    // N-point transform of the thread's points, in and out.  The two buffers alternate, so one barrier per
-    // exchange: a buffer is written again only after the barrier that follows the reads of it.
-    template <bool INV> __device__ __forceinline__ void dft(float2 (&v)[E]) {
-        DFT<4, INV>::run(v);
-        float2* a = s + buf;
-#pragma unroll
-        for (int r = 0; r < E; ++r) a[slot(4 * j + r, line)] = v[r];
-        __syncthreads();
-        mid<RM, 4, INV>(w1);
-        if constexpr (P::S == 4) mid<4, 16, INV>(w2);
-        const float2* b = s + buf;
-        buf = lds_half<N>() - buf;
-#pragma unroll
-        for (int r = 0; r < E; ++r) v[r] = b[slot(j + r * T, line)];
-#pragma unroll
-        for (int r = 1; r < E; ++r) v[r] = INV ? cmulc(v[r], w3[r - 1]) : cmul(v[r], w3[r - 1]);
-        DFT<4, INV>::run(v);
-    }
-};
 
 // sum of one double per thread over the workgroup, in the first thread
 template <int NT> __device__ __forceinline__ double group_sum(double v, double* red) {
@@ -147,10 +67,12 @@ template <int NT> __device__ __forceinline__ double group_sum(double v, double* 
 enum { PROBE, SHIFT, FIRST, FWD, LAST, EXIT, ADJ, BACK, STEP };
 
 template <int N, int KIND, bool COL> __global__ __launch_bounds__(N) void k_line_pass(LineArgs A) {
-    constexpr int N2 = N * N, T = N / E, G = N / TL;
-    __shared__ float2 s[2 * lds_half<N>()];
+    using F_ = Line<N, TL>;
+    constexpr int N2 = N * N, E = F_::E, T = F_::T, G = N / TL;
+    static_assert(F_::NT == N, "launched with N threads");
+    __shared__ float2 s[F_::LDS_ELEMS];
     __shared__ double red[(N + 63) / 64];
-    Line<N> F;
+    F_ F;
     F.init(s, A.tw);
     const int line = blockIdx.x * TL + F.line, j = F.j;
     // index of point r of the thread in arrays with contiguous lines, and in arrays of the other orientation

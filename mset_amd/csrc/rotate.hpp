@@ -9,6 +9,8 @@ namespace mset {
 struct RotWork {
     float2* w = nullptr;              // complex work volume
     size_t wn = 0;
+    float* nyq = nullptr;             // planar rotations: Nyquist component along the third axis
+    size_t nn = 0;
     std::map<int, float2*> tw;        // twiddle tables by line length
 };
 
@@ -23,8 +25,8 @@ bool rot_size_supported(int n);
 bool rot_matrix(const double* v1, const double* v2, const double* v3, double phi, double theta, double psi,
                 bool inverse, double R[9]);
 ShearPlan plan_rotation(const double R[9], double rot_step_init);
-// In-place rotation of a device volume float[nz][ny][nx]; returns an MSET_* status.
-int rot_run(RotWork& W, float* vol, int nx, int ny, int nz, const double R[9], double rot_step_init, hipStream_t st);
+// vol = rotation of src, device volumes float[nz][ny][nx] (src may be vol); returns an MSET_* status.
+int rot_run(RotWork& W, const float* src, float* vol, int nx, int ny, int nz, const double R[9], double rot_step_init, hipStream_t st);
 const char* rot_last_error();
 void rot_release(RotWork& W);
 
