@@ -140,7 +140,7 @@ hipError_t launch_update_volume(float* V, const float* G, int n, int nz, int bin
 hipError_t launch_update_positions(float* x, float* y, const float* dpos, int npos, float s3, hipStream_t st);
 hipError_t launch_positivity(float* V, size_t n, hipStream_t st);
 
-// total-variation regulariser (tv.hip): dual field (3 volumes) + scratch volume, reduction partials
+// total-variation regulariser (tv.hip): two dual fields (3 volumes each) + f / lambda, reduction partials
 struct TvWork {
     float* P = nullptr;
     double* part = nullptr;
