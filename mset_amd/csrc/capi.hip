@@ -86,6 +86,7 @@ using ProfMap = std::map<std::string, Prof>;
 struct Workspace {
     DevBuf<float2> save, trans, probeF, pslab, PG, planes, lines;
     DevBuf<float> gslab, G;
+    DevBuf<float> io;                        // volume of a host-to-host call (mset_rotate, mset_tv), kept between calls
     int exit_waves = MSET_EXIT_WAVES_AUTO;   // requested exit-wave variant of the batched kernels
     int slot_limit = 0;                      // cap on the persistent grid of the batched kernels (0: none)
     int engine = MSET_ENGINE_AUTO;           // MSET_ENGINE_* flags: plane routine at 256, workgroup shape
@@ -700,7 +701,10 @@ struct mset_recon {
     std::vector<float> prop_host;
     std::vector<mset_ctx*> tilts;
     std::vector<std::array<double, 3>> angles;
-    std::vector<std::vector<float>> snap_probe, snap_x, snap_y;
+    // the snapshot of every tilt's probe and positions, one after another
+    DevBuf<float2> probe_snap;
+    DevBuf<float> pos_snap;
+    std::vector<int> snap_npos;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int graph_key[3] = {-1, -1, -1};
@@ -1021,7 +1025,7 @@ int mset_rotate(mset_ctx* c, const float* in, float* out, int nx, int ny, int nz
     if (!rot_size_supported(nx) || !rot_size_supported(ny) || !rot_size_supported(nz))
         return fail(MSET_EUNSUPPORTED, "rotation line length not built");
     const size_t nv = (size_t)nx * ny * nz;
-    DevBuf<float> buf;
+    DevBuf<float>& buf = c->ws->io;
     CHK(buf.ensure(nv, "rotation volume"));
     HIPCHK(hipMemcpyAsync(buf.p, in, sizeof(float) * nv, hipMemcpyHostToDevice, c->stream));
     {
@@ -1084,7 +1088,7 @@ int mset_tv(mset_ctx* c, const float* in, float* out, int nx, int ny, int nz, fl
     if (nx <= 0 || ny <= 0 || nz <= 0) return fail(MSET_EINVAL, "sizes must be positive");
     if (!(lambda > 0.f) || n_iter < 0) return fail(MSET_EINVAL, "TV needs lambda > 0 and n_iter >= 0");
     const long long nv = (long long)nx * ny * nz;
-    DevBuf<float> buf;
+    DevBuf<float>& buf = c->ws->io;
     CHK(buf.ensure((size_t)nv, "TV volume"));
     if (tv_ensure(c->ws->tv, nv) != 0) return fail(MSET_ENOMEM, "hipMalloc: TV work");
     HIPCHK(hipMemcpyAsync(buf.p, in, sizeof(float) * nv, hipMemcpyHostToDevice, c->stream));
@@ -1384,40 +1388,46 @@ int mset_recon_set_engine(mset_recon* r, int engine) {
     return MSET_OK;
 }
 
-int mset_recon_snapshot(mset_recon* r) {
-    CHK(check_recon(r));
+// copies between the snapshot and the state, on the device
+static int snapshot_copy(mset_recon* r, bool save) {
     const size_t n2 = (size_t)r->n * r->n, nv = n2 * r->nz;
-    CHK(r->rec_snap.ensure(nv, "snapshot"));
-    HIPCHK(hipMemcpyAsync(r->rec_snap.p, r->rec.p, sizeof(float) * nv, hipMemcpyDeviceToDevice, r->stream));
-    r->snap_probe.resize(r->tilts.size());
-    r->snap_x.resize(r->tilts.size());
-    r->snap_y.resize(r->tilts.size());
+    auto copy = [&](void* state, void* snap, size_t bytes) {
+        return hipMemcpyAsync(save ? snap : state, save ? state : snap, bytes, hipMemcpyDeviceToDevice, r->stream);
+    };
+    HIPCHK(copy(r->rec.p, r->rec_snap.p, sizeof(float) * nv));
+    size_t off = 0;
     for (size_t j = 0; j < r->tilts.size(); ++j) {
         mset_ctx* c = r->tilts[j];
-        r->snap_probe[j].resize(2 * n2);
-        r->snap_x[j].resize(c->npos);
-        r->snap_y[j].resize(c->npos);
-        HIPCHK(hipMemcpyAsync(r->snap_probe[j].data(), c->probe.p, sizeof(float2) * n2, hipMemcpyDeviceToHost, r->stream));
-        HIPCHK(hipMemcpyAsync(r->snap_x[j].data(), c->x.p, sizeof(float) * c->npos, hipMemcpyDeviceToHost, r->stream));
-        HIPCHK(hipMemcpyAsync(r->snap_y[j].data(), c->y.p, sizeof(float) * c->npos, hipMemcpyDeviceToHost, r->stream));
+        HIPCHK(copy(c->probe.p, r->probe_snap.p + n2 * j, sizeof(float2) * n2));
+        const size_t had = r->snap_npos[j];       // positions when the snapshot was taken, at least c->npos
+        HIPCHK(copy(c->x.p, r->pos_snap.p + off, sizeof(float) * c->npos));
+        HIPCHK(copy(c->y.p, r->pos_snap.p + off + had, sizeof(float) * c->npos));
+        off += 2 * had;
     }
     HIPCHK(hipStreamSynchronize(r->stream));
     return MSET_OK;
 }
 
+int mset_recon_snapshot(mset_recon* r) {
+    CHK(check_recon(r));
+    const size_t n2 = (size_t)r->n * r->n;
+    CHK(r->rec_snap.ensure(n2 * r->nz, "snapshot"));
+    CHK(r->probe_snap.ensure(n2 * r->tilts.size(), "snapshot"));
+    size_t tot = 0;
+    for (const mset_ctx* c : r->tilts) tot += c->npos;
+    CHK(r->pos_snap.ensure(2 * tot, "snapshot"));
+    r->snap_npos.clear();
+    for (const mset_ctx* c : r->tilts) r->snap_npos.push_back(c->npos);
+    return snapshot_copy(r, true);
+}
+
 int mset_recon_restore(mset_recon* r) {
     CHK(check_recon(r));
     if (!r->rec_snap.p) return fail(MSET_EINVAL, "no snapshot taken");
-    const size_t n2 = (size_t)r->n * r->n, nv = n2 * r->nz;
-    HIPCHK(hipMemcpyAsync(r->rec.p, r->rec_snap.p, sizeof(float) * nv, hipMemcpyDeviceToDevice, r->stream));
-    for (size_t j = 0; j < r->tilts.size(); ++j) {
-        mset_ctx* c = r->tilts[j];
-        HIPCHK(hipMemcpyAsync(c->probe.p, r->snap_probe[j].data(), sizeof(float2) * n2, hipMemcpyHostToDevice, r->stream));
-        HIPCHK(hipMemcpyAsync(c->x.p, r->snap_x[j].data(), sizeof(float) * c->npos, hipMemcpyHostToDevice, r->stream));
-        HIPCHK(hipMemcpyAsync(c->y.p, r->snap_y[j].data(), sizeof(float) * c->npos, hipMemcpyHostToDevice, r->stream));
-    }
-    HIPCHK(hipStreamSynchronize(r->stream));
-    return MSET_OK;
+    for (size_t j = 0; j < r->tilts.size(); ++j)
+        if (r->snap_npos[j] < r->tilts[j]->npos)
+            return fail(MSET_EINVAL, "tilt " + std::to_string(j) + " has more positions than the snapshot");
+    return snapshot_copy(r, false);
 }
 
 int mset_recon_profile_enable(mset_recon* r, int enable) {

@@ -70,9 +70,9 @@ template <int W> struct Row {
 // One iteration, W elements of a row per thread (4 where rows are whole float4s): the residual D of the elements
 // and of their x, y and z successors is formed from P (25 loads for 4 elements, all but 7 of them hits in
 // L1 or L2, requested together), so D is never stored and P, q are read once and P written once: 28 bytes of
-// memory traffic per element instead of 48 in two launches with a stored D.  q = f / lambda is formed once, since a
-// division per element and iteration costs more than everything else here.  The fields alternate between Pi
-// and Po.  64 x 128 x 128 volume: 13.8 us per iteration as two launches with 64-bit index divisions.
+// memory traffic per element instead of 48 in two launches with a stored D.  q = f / lambda is formed once.  The
+// fields alternate between Pi and Po.  64 x 128 x 128 volume: 13.8 us per iteration as two launches with 64-bit
+// index divisions, 8.3 us now, bound by the 29 MB that a launch reads from and writes back past L2.
 // I: index type, 32-bit unless the volume needs more (64-bit divisions cost more than the stencil).
 template <int W, class I>
 __global__ __launch_bounds__(256) void k_tv_iterate(int nx, int ny, int nz, const float* __restrict__ Pi,

@@ -79,7 +79,8 @@ def footprint_bytes(spec, slots):
     n2 = spec.P * spec.P
     nv = n2 * spec.vol
     L, nt, npos = spec.L, len(spec.tilts), spec.scan * spec.scan
-    per_tilt = nv * 4 + npos * n2 * 4 * 2 + n2 * 8 * 2 + npos * 24     # V, patterns (+ staging), probe, prop
+    # V, patterns (+ staging), probe (+ snapshot), prop, positions (+ snapshot)
+    per_tilt = nv * 4 + npos * n2 * 4 * 2 + n2 * 8 * 3 + npos * 32
     shared = (slots * (L + 2) * n2 * 8 + slots * L * n2 * 4 + slots * n2 * 8 + L * n2 * 8 * 2 + n2 * 24
               + nv * 8 * 2)                                            # save, gslab, pslab, trans, G, rotation
     if spec.P >= 256:
