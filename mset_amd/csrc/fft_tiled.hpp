@@ -116,6 +116,21 @@ template <int N, int NT_> struct TiledEngine {
         XS = PB + N * N;
     }
 
+    // The LDS tile s[pos][line] out to dst along the other axis, element (line l0 + l, position pos) at
+    // dst[(l0 + l) N + pos]: TL N = R NT elements, the thread's R all read before the first is stored.  (As a loop
+    // from threadIdx.x the compiler did not unroll it, an LDS latency per element: 12.95 ms per batched launch of 512
+    // positions x 32 planes, 12.46 now; with 64-bit addresses instead of a buffer view 12.78, 80 more spilled registers.)
+    __device__ __forceinline__ void store_other(float2* dst, int l0) const {
+        static_assert(NT % N == 0 && TL * N == R * NT, "a thread keeps its position");
+        const int pos = threadIdx.x % N, l = threadIdx.x / N;
+        const BufC d(dst + l0 * N, TL * N);
+        float2 q[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) q[i] = s[pos * TP + l + i * (NT / N)];
+#pragma unroll
+        for (int i = 0; i < R; ++i) d.put(Idx{(unsigned)(l * N + pos), (unsigned)(i * NT)}, q[i]);
+    }
+
     // 256-point transform of the thread's elements j + 16 r (r < 16) of line `line`, in and out; LEAD: the
     // LDS may still be read by other threads (a transform earlier in the same tile) and needs a barrier
     template <int D, bool LEAD> __device__ __forceinline__ void dft(float2 (&v)[R], int line, int j) {
@@ -183,10 +198,7 @@ template <int N, int NT_> struct TiledEngine {
 #pragma unroll
                 for (int r = 0; r < R; ++r) s[(j + R * r) * TP + line] = v[r];
                 __syncthreads();
-                for (int e = t; e < TL * N; e += NT) {
-                    const int pos = e % N, l = e / N;
-                    out[(l0 + l) * N + pos] = s[pos * TP + l];
-                }
+                store_other(out, l0);
             } else {
 #pragma unroll
                 for (int r = 0; r < R; ++r) out[(j + R * r) * N + ln] = v[r];
@@ -300,8 +312,9 @@ template <int N, int NT_> struct TiledEngine {
                 for (int r = 0; r < R; ++r) v[r] = make_float2(0.f, 0.f);
                 pre.template run<COL>(*this, v, l0, line, j);
             } else {
+                const BufC ib(in + l0, N * N - l0);
 #pragma unroll
-                for (int r = 0; r < R; ++r) v[r] = in[(j + R * r) * N + l0 + line];
+                for (int r = 0; r < R; ++r) v[r] = ib[Idx{(unsigned)(j * N + line), (unsigned)(R * r * N)}];
                 step<COL>(pre, v, l0, line, j);
             }
             if constexpr (D1 != NONE) dft<D1, PRE_TILE>(v, line, j);
@@ -326,10 +339,7 @@ template <int N, int NT_> struct TiledEngine {
 #pragma unroll
                 for (int r = 0; r < R; ++r) s[(j + R * r) * TP + line] = v[r];
                 __syncthreads();
-                for (int e = t; e < TL * N; e += NT) {
-                    const int pos = e % N, l = e / N;
-                    out[(l0 + l) * N + pos] = s[pos * TP + l];
-                }
+                store_other(out, l0);
             }
             __syncthreads();
         }
@@ -344,18 +354,17 @@ template <int N, int NT_> struct TiledEngine {
 #pragma unroll
         for (int r = 0; r < R; ++r) s[(j + R * r) * TP + line] = v[r];
         __syncthreads();
-        for (int e = threadIdx.x; e < TL * N; e += NT) {
-            const int pos = e % N, l = e / N;
-            dst[(l0 + l) * N + pos] = s[pos * TP + l];
-        }
+        store_other(dst, l0);
     }
     template <class T> __device__ __forceinline__ void other_to_tile(const T* src, T (&o)[R], int l0, int line, int j) {
         __syncthreads();
         T* st = reinterpret_cast<T*>(s);   // T is float or float2: at most one float2 per LDS slot
-        for (int e = threadIdx.x; e < TL * N; e += NT) {
-            const int pos = e % N, l = e / N;
-            st[(pos * TP + l) * (sizeof(float2) / sizeof(T))] = src[(l0 + l) * N + pos];
-        }
+        const int pos = threadIdx.x % N, l = threadIdx.x / N;
+        T q[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) q[i] = src[(l0 + l + i * (NT / N)) * N + pos];
+#pragma unroll
+        for (int i = 0; i < R; ++i) st[(pos * TP + l + i * (NT / N)) * (sizeof(float2) / sizeof(T))] = q[i];
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < R; ++r) o[r] = st[((j + R * r) * TP + line) * (sizeof(float2) / sizeof(T))];
