@@ -8,7 +8,7 @@ import subprocess
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = ['batch_store.hip', 'batch_variants.hip', 'multislice.hip', 'forward.hip', 'line_passes.hip', 'elementwise.hip',
+SOURCES = ['batch_store.hip', 'batch_variants.hip', 'multislice.hip', 'forward.hip', 'line_passes.hip', 'sep_lines.hip', 'elementwise.hip',
            'rotate.hip', 'tv.hip', 'capi.hip']
 LIB = os.path.join(HERE, 'libmset_amd.so')
 # stand-alone counter-calibration program (known-size copies for rocprofv3's FETCH_SIZE / WRITE_SIZE)

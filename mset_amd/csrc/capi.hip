@@ -286,18 +286,33 @@ bool sep_batch(const mset_ctx* c) {
     return sep_fwd(c) && c->p.grad_mode == GRAD_REF && (c->ws->waves == WAVES_STORE || c->ws->waves == WAVES_CHECKPOINT);
 }
 
+// The on-chip separable routine (sep_lines.hpp): forward-only launches below 256, gradients and the one-position
+// kernel with the reference pairing and stored waves below 128.  12 planes, the LDS engine against it, gradient
+// and forward-only: 256 positions 43 -> 35 and 24 -> 18 us at 16, 67 -> 63 and 35 -> 30 at 24, 73 -> 63 and 37 -> 33 at
+// 32, 131 -> 94 and 65 -> 41 at 48, 167 -> 132 and 74 -> 49 at 64, 440 -> 330 and 181 -> 121 at 96; 1400 positions
+// 54 -> 43, 137 -> 115, 167 -> 156, 652 -> 413, 787 -> 673 us (700 at 96: 1286 -> 995).  At 128, 16 planes, 1024 positions:
+// forward-only 1188 -> 958 us against the register engine, the gradient 2838 -> 2846 (its operands leave too few
+// registers), so that stays there.
+bool sep_fwd_lines(const mset_ctx* c) {
+    return c->n <= 128 && c->prop_sep && !sset(c) && !(c->ws->engine & MSET_ENGINE_GENERAL);
+}
+bool sep_grad_lines(const mset_ctx* c) { return c->n < 128 && sep_fwd_lines(c) && c->p.grad_mode == GRAD_REF; }
+constexpr int SHAPE_SEP = 3;   // its place among the workgroup shapes of a batched call
+
 // workgroup shape of a batched call: the alternative shape (MSET_ENGINE_ALT_SHAPE) exists for stored waves; a
 // gradient request (fixed) takes it below 128 as well, see Cfg
 int shape_for(const mset_ctx* c, int waves, bool fixed) {
     const bool alt = (c->ws->engine & MSET_ENGINE_ALT_SHAPE) || (fixed && c->n < 128 && c->n != 48);
-    return alt && waves == WAVES_STORE ? 1 : 0;
+    if (alt || waves != WAVES_STORE) return waves == WAVES_STORE ? 1 : 0;
+    return sep_grad_lines(c) && !fixed ? SHAPE_SEP : 0;
 }
 
 // workgroups of the batched kernel of a workgroup shape the device keeps resident at once (1 per CU at
 // N = 128 in the default shape); by default the shape of the last batched call
 int device_slots(mset_ctx* c, int shape) {
     int per_cu = 1;
-    if (occupancy_batch(c->n, shape, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
+    const hipError_t e = shape == SHAPE_SEP ? occupancy_sep(c->n, false, &per_cu) : occupancy_batch(c->n, shape, &per_cu);
+    if (e != hipSuccess || per_cu < 1) per_cu = 1;
     return c->cus * per_cu;
 }
 int device_slots(mset_ctx* c) { return device_slots(c, c->ws->shape); }
@@ -439,9 +454,9 @@ int read_errors(mset_ctx* c, int first, int count, double* out) {
 }
 
 // The sequential path as line passes over the whole device (line_passes.hip): a separable propagator, the
-// reference pairing, 64 x 64 and up.  Both ways cost about the same per plane at any depth; per position,
-// one workgroup against line passes: 137 and 71 us at 64 x 64 (6 planes), 576 and 205 us at 128 x 128 (16),
-// 4.5 ms and 0.45 ms at 256 x 256 (32).
+// reference pairing, from 96 x 96 up.  Both ways cost about the same per plane at any depth; per position, one
+// workgroup of the on-chip separable routine against line passes: 71 and 70 us at 64 x 64 (6 planes; 149 and 159
+// with 16), 166 and 91 us at 96 x 96 (6), 267 and 94 us at 128 x 128 (6).
 bool plain_lines(const mset_ctx* c) {
     return position_lines_supported(c->n) && c->prop_sep && !sset(c) && c->p.grad_mode == GRAD_REF &&
            !(c->ws->engine & MSET_ENGINE_GENERAL);
@@ -463,18 +478,31 @@ int issue_plain(mset_ctx* c) {
     CHK(c->ws->gslab.ensure((size_t)c->L * plane(c), "gradient planes"));
     PosArgs A = base_args(c);
     const float s1 = c->p.step_size[0];
+    const bool sep = sep_grad_lines(c);
+    // transmission planes from the current volume, the position, then its object step, which also forms the next
+    // position's transmission (STEP02_FORWARD_4D.m:12-20, STEP03_BACK.m:84): the volume passes run on the whole
+    // device
+    HIPCHK(launch_transmission(c->V.p, c->ws->trans.p, c->n, c->nz, binning(c), sset(c) ? 1 : 0, c->p.sigma,
+                               c->p.potential_pixelsize, c->stream));
     for (int k = 0; k < c->npos; ++k) {
-        // transmission planes from the current volume, the position, then its object step
-        // (STEP02_FORWARD_4D.m:12-20, STEP03_BACK.m:84): the volume passes run on the whole device
-        HIPCHK(launch_transmission(c->V.p, c->ws->trans.p, c->n, c->nz, binning(c), sset(c) ? 1 : 0, c->p.sigma,
-                                   c->p.potential_pixelsize, c->stream));
         {
             Timed t(c, "position_plain");
-            HIPCHK(launch_plain(c->n, A, k, c->stream));
+            if (sep) HIPCHK(launch_sep_plain(c->n, A, k, c->stream));
+            else HIPCHK(launch_plain(c->n, A, k, c->stream));
         }
-        if (s1 != 0.f) HIPCHK(launch_update_volume(c->V.p, c->ws->gslab.p, c->n, c->nz, binning(c), s1, c->stream));
+        if (s1 != 0.f)
+            HIPCHK(launch_update_volume(c->V.p, c->ws->gslab.p, c->n, c->nz, binning(c), s1, c->stream, c->ws->trans.p,
+                                        sset(c) ? 1 : 0, c->p.sigma, c->p.potential_pixelsize));
     }
     return MSET_OK;
+}
+
+// grid of the forward-only on-chip separable kernel: the resident workgroups, capped by the slot limit
+int fwd_slots(const mset_ctx* c) {
+    int per_cu = 1;
+    if (occupancy_sep(c->n, true, &per_cu) != hipSuccess || per_cu < 1) per_cu = 1;
+    const int s = c->cus * per_cu;
+    return c->ws->slot_limit > 0 ? std::min(s, c->ws->slot_limit) : s;
 }
 
 int issue_fwd(mset_ctx* c, float* inten) {
@@ -486,7 +514,8 @@ int issue_fwd(mset_ctx* c, float* inten) {
     A.count = c->npos;
     A.inten = inten;
     Timed t(c, "position_fwd");
-    HIPCHK(launch_fwd(c->n, A, plane_in_global(c->n) ? batch_slots(c) : batch_slots(c, 0), fwd_shape(c, c->npos), c->stream));
+    if (sep_fwd_lines(c)) HIPCHK(launch_sep_fwd(c->n, A, std::min(fwd_slots(c), c->npos), false, c->stream));
+    else HIPCHK(launch_fwd(c->n, A, plane_in_global(c->n) ? batch_slots(c) : batch_slots(c, 0), fwd_shape(c, c->npos), c->stream));
     return MSET_OK;
 }
 
@@ -510,7 +539,8 @@ int issue_grad(mset_ctx* c, int first, int count, bool apply, int want) {
     // every used slab receives at least one position, and its first one writes it
     {
         Timed t(c, "position_batch");
-        HIPCHK(launch_batch(c->n, A, grid, batch_shape(c, W.shape, sep, W.waves, count, !apply), c->stream));
+        if (W.shape == SHAPE_SEP) HIPCHK(launch_sep_batch(c->n, A, grid, c->stream));
+        else HIPCHK(launch_batch(c->n, A, grid, batch_shape(c, W.shape, sep, W.waves, count, !apply), c->stream));
     }
     HIPCHK(launch_reduce_slabs(W.gslab.p, used, (size_t)planes(c) * plane(c), W.G.p, c->stream));
     if (sep) HIPCHK(launch_untranspose_odd(W.G.p, c->n, c->L, c->stream));
@@ -734,9 +764,8 @@ int check_recon(mset_recon* r) {
 }
 
 // A sequential pass in more launches than this is issued eagerly even when a graph is asked for: a captured
-// pass has a node per launch, and the host issues the launches faster than they run except at the smallest
-// plane of the line passes (3 tilts of 64 positions: 13.8 ms eager, 12.2 ms replayed at 64 x 64, 3.5k launches;
-// 16.6 and 16.5 ms at 128 x 128, 3.5k launches).
+// pass has a node per launch, and the host issues the launches faster than they run (3 tilts of 64 positions at
+// 128 x 128, 3.5k launches: 16.6 ms eager, 16.5 ms replayed).
 constexpr size_t PLAIN_GRAPH_LAUNCHES = 65536;
 
 size_t plain_launches(const mset_recon* r) {
@@ -1304,7 +1333,8 @@ int mset_recon_error_pass(mset_recon* r, double* errs) {
     A.sep = sep ? 1 : 0;
     {
         Timed t(c0, "position_fwd");
-        HIPCHK(launch_fwd_tilts(r->n, A, grid, fwd_shape(c0, (int)std::min<size_t>(tot, INT_MAX)), r->stream));
+        if (sep_fwd_lines(c0)) HIPCHK(launch_sep_fwd(r->n, A, (int)std::min<size_t>(fwd_slots(c0), tot), true, r->stream));
+        else HIPCHK(launch_fwd_tilts(r->n, A, grid, fwd_shape(c0, (int)std::min<size_t>(tot, INT_MAX)), r->stream));
     }
     std::vector<double> e(tot);
     HIPCHK(hipMemcpyAsync(e.data(), r->err_all.p, sizeof(double) * tot, hipMemcpyDeviceToHost, r->stream));

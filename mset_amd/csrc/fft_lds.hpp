@@ -160,6 +160,36 @@ template <bool INV> struct DFT<6, INV> {
     }
 };
 
+// 12 = 3 x 4: four-point transforms over n1 + 3 n2, twiddles W_12^(n1 k1), three-point transforms
+template <bool INV> struct DFT<12, INV> {
+    __device__ __forceinline__ static void run(float2* v) {
+        constexpr float h = 0.86602540378443865f;
+        float2 u[3][4];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) u[a][b] = v[a + 3 * b];
+            DFT<4, INV>::run(u[a]);
+        }
+        const float2 w1 = make_float2(h, INV ? 0.5f : -0.5f), w2 = make_float2(0.5f, INV ? h : -h);
+        const float2 w4 = make_float2(-0.5f, INV ? h : -h);
+        u[1][1] = cmul(u[1][1], w1);
+        u[1][2] = cmul(u[1][2], w2);
+        u[1][3] = mul_mi<INV>(u[1][3]);
+        u[2][1] = cmul(u[2][1], w2);
+        u[2][2] = cmul(u[2][2], w4);
+        u[2][3] = make_float2(-u[2][3].x, -u[2][3].y);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float2 t[3] = {u[0][k], u[1][k], u[2][k]};
+            DFT<3, INV>::run(t);
+            v[k] = t[0];
+            v[k + 4] = t[1];
+            v[k + 8] = t[2];
+        }
+    }
+};
+
 // ------------------------------------------------------------------ element points and buffer views
 // An element as the engines hand it to functors: its coordinates and its index in the layout the
 // current orientation streams (row-major [y][x] when consecutive lanes run along x, transposed [x][y]

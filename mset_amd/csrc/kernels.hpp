@@ -123,6 +123,12 @@ hipError_t launch_plane_fft(int n, const float2* in, float2* out, const float2* 
                             float beta2 = 0.f);
 bool plane_in_global(int n);     // the position kernels keep the plane in global memory (planes buffer)
 hipError_t occupancy_batch(int n, int shape, int* blocks_per_cu);
+// on-chip separable routine (sep_lines.hip): A.pfac, the multislice operator; forward-only up to 128, below it the
+// gradient kernels with the reference pairing and stored waves.  launch_sep_plain: as launch_plain.
+hipError_t launch_sep_batch(int n, const PosArgs& A, int grid, hipStream_t st);
+hipError_t launch_sep_plain(int n, const PosArgs& A, int k, hipStream_t st);
+hipError_t launch_sep_fwd(int n, const PosArgs& A, int grid, bool tilts, hipStream_t st);
+hipError_t occupancy_sep(int n, bool fwd, int* blocks_per_cu);
 
 // element-wise kernels (elementwise.hip)
 hipError_t launch_ingest_patterns(const float* M, float* sqrtM, int n, long long npos, int transpose, hipStream_t st);
@@ -136,7 +142,9 @@ hipError_t launch_transmission_sep(const float* V, float* Tf, float* Tb, int n, 
 hipError_t launch_untranspose_odd(float* G, int n, int L, hipStream_t st);
 hipError_t launch_reduce_slabs(const float* slab, int nslab, size_t n, float* out, hipStream_t st);
 hipError_t launch_reduce_cslabs(const float2* slab, int nslab, size_t n, float2* out, hipStream_t st);
-hipError_t launch_update_volume(float* V, const float* G, int n, int nz, int bin, float s1, hipStream_t st);
+// V[z] += s1 G[bin of z]; with trans also the transmission planes of the updated volume (as launch_transmission)
+hipError_t launch_update_volume(float* V, const float* G, int n, int nz, int bin, float s1, hipStream_t st,
+                                float2* trans = nullptr, int sset = 0, float sigma = 0.f, float dx = 0.f);
 hipError_t launch_update_positions(float* x, float* y, const float* dpos, int npos, float s3, hipStream_t st);
 hipError_t launch_positivity(float* V, size_t n, hipStream_t st);
 

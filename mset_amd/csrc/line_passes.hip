@@ -33,9 +33,9 @@
 // it again, so there are no transmission planes, gradient planes or update launches.  Waves, loss and
 // position sums, rounding order of the transmission and the update as in process_position.
 //
-// Measured per position, before as one workgroup and now: 137 -> 71 us at 64 x 64 x 6 planes (18 launches),
-// 576 -> 205 us at 128 x 128 x 16 (38), 4.5 -> 0.45 ms at 256 x 256 x 32 (70); a pass with four transforms takes
-// 5 to 6 us at 128, about 2 of them the launch and the loads.
+// Measured per position, before as one workgroup and now: 576 -> 205 us at 128 x 128 x 16 planes (38 launches),
+// 4.5 -> 0.45 ms at 256 x 256 x 32 (70); a pass with four transforms takes 5 to 6 us at 128, about 2 of them the
+// launch and the loads.
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
@@ -379,14 +379,13 @@ template <int N> hipError_t position_lines(const PosArgs& P, int k, float2* work
 
 }  // namespace
 
-bool position_lines_supported(int n) { return n == 64 || n == 96 || n == 128 || n == 256; }
+bool position_lines_supported(int n) { return n == 96 || n == 128 || n == 256; }
 
 // two plane buffers, the shift factors and three sums per workgroup
 size_t position_lines_work(int n) { return 2 * (size_t)n * n + 2 * (size_t)n + 3 * (size_t)(n / TL); }
 
 hipError_t launch_position_lines(int n, const PosArgs& P, int k, float2* work, hipStream_t st) {
     switch (n) {
-        case 64: return position_lines<64>(P, k, work, st);
         case 96: return position_lines<96>(P, k, work, st);
         case 128: return position_lines<128>(P, k, work, st);
         case 256: return position_lines<256>(P, k, work, st);

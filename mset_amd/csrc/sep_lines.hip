@@ -1,0 +1,50 @@
+// sep_lines.hip -- launchers of the on-chip separable routine (sep_lines.hpp).
+#include "sep_lines.hpp"
+
+namespace mset {
+
+#define MSET_SEP_DISPATCH(N, BODY)                           \
+    switch (N) {                                             \
+        case 16: { constexpr int NN = 16; BODY; } break;     \
+        case 24: { constexpr int NN = 24; BODY; } break;     \
+        case 32: { constexpr int NN = 32; BODY; } break;     \
+        case 48: { constexpr int NN = 48; BODY; } break;     \
+        case 64: { constexpr int NN = 64; BODY; } break;     \
+        case 96: { constexpr int NN = 96; BODY; } break;     \
+        default: return hipErrorInvalidValue;                \
+    }
+
+hipError_t launch_sep_batch(int n, const PosArgs& A, int grid, hipStream_t st) {
+    if (!A.pfac || A.sset || A.grad_mode != GRAD_REF || A.waves != WAVES_STORE) return hipErrorInvalidValue;
+    MSET_SEP_DISPATCH(n, hipLaunchKernelGGL((k_sep_batch<NN>), dim3(grid), dim3(SepCfg<NN>::NT), 0, st, A))
+    return hipGetLastError();
+}
+
+hipError_t launch_sep_plain(int n, const PosArgs& A, int k, hipStream_t st) {
+    if (!A.pfac || A.sset || A.grad_mode != GRAD_REF) return hipErrorInvalidValue;
+    MSET_SEP_DISPATCH(n, hipLaunchKernelGGL((k_sep_plain<NN>), dim3(1), dim3(SepCfg<NN>::NT), 0, st, A, k))
+    return hipGetLastError();
+}
+
+hipError_t launch_sep_fwd(int n, const PosArgs& A, int grid, bool tilts, hipStream_t st) {
+    if (!A.pfac || A.sset) return hipErrorInvalidValue;
+#define MSET_FWD(N)                                                                                             \
+    if (tilts) hipLaunchKernelGGL((k_sep_fwd<N, true>), dim3(grid), dim3(SepCfg<N>::NT), 0, st, A);             \
+    else hipLaunchKernelGGL((k_sep_fwd<N, false>), dim3(grid), dim3(SepCfg<N>::NT), 0, st, A)
+    if (n == 128) {
+        MSET_FWD(128);
+    } else {
+        MSET_SEP_DISPATCH(n, MSET_FWD(NN))
+    }
+#undef MSET_FWD
+    return hipGetLastError();
+}
+
+hipError_t occupancy_sep(int n, bool fwd, int* per_cu) {
+    if (fwd && n == 128) return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, (k_sep_fwd<128, false>), SepCfg<128>::NT, 0);
+    if (fwd) MSET_SEP_DISPATCH(n, return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, (k_sep_fwd<NN, false>), SepCfg<NN>::NT, 0))
+    MSET_SEP_DISPATCH(n, return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, (k_sep_batch<NN>), SepCfg<NN>::NT, 0))
+    return hipSuccess;
+}
+
+}  // namespace mset

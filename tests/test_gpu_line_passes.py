@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 # every plane size; odd and even plane counts (the orientation of the exit pass), one plane, a bin above the
 # four slices kept in registers, partial last bins, and each step alone (launches left out)
 @pytest.mark.parametrize('n,nz,binning,steps', [
-    (64, 1, 1, (30.0, 2e-3, 2e-2)), (64, 13, 6, (30.0, 2e-3, 2e-2)), (96, 8, 4, (30.0, 2e-3, 2e-2)),
+    (64, 1, 1, (30.0, 2e-3, 2e-2)), (64, 13, 6, (30.0, 2e-3, 2e-2)), (96, 1, 1, (30.0, 2e-3, 2e-2)),
+    (128, 13, 6, (30.0, 2e-3, 2e-2)), (96, 8, 4, (30.0, 2e-3, 2e-2)),
     (96, 5, 3, (30.0, 0.0, 2e-2)), (128, 11, 5, (30.0, 2e-3, 0.0)), (128, 6, 2, (0.0, 0.0, 0.0)),
     (256, 3, 2, (30.0, 2e-3, 2e-2)), (256, 2, 2, (0.0, 2e-3, 2e-2))])
 def test_line_passes_vs_oracle(n, nz, binning, steps):
