@@ -299,11 +299,12 @@ bool sep_fwd_lines(const mset_ctx* c) {
 bool sep_grad_lines(const mset_ctx* c) { return c->n < 128 && sep_fwd_lines(c) && c->p.grad_mode == GRAD_REF; }
 constexpr int SHAPE_SEP = 3;   // its place among the workgroup shapes of a batched call
 
-// workgroup shape of a batched call: the alternative shape (MSET_ENGINE_ALT_SHAPE) exists for stored waves; a
-// gradient request (fixed) takes it below 128 as well, see Cfg
+// Workgroup shape of a batched call: the alternative shape (MSET_ENGINE_ALT_SHAPE) exists for stored waves.  A
+// gradient request (fixed) stays on the general routine: the two routines' waves differ by 1e-6, which position
+// terms that cancel turn into 1e-4 of a gradient, and gradients are what callers difference.
 int shape_for(const mset_ctx* c, int waves, bool fixed) {
-    const bool alt = (c->ws->engine & MSET_ENGINE_ALT_SHAPE) || (fixed && c->n < 128 && c->n != 48);
-    if (alt || waves != WAVES_STORE) return waves == WAVES_STORE ? 1 : 0;
+    if (waves != WAVES_STORE) return 0;
+    if (c->ws->engine & MSET_ENGINE_ALT_SHAPE) return 1;
     return sep_grad_lines(c) && !fixed ? SHAPE_SEP : 0;
 }
 
@@ -334,18 +335,17 @@ int grad_slabs(mset_ctx* c, int shape) { return std::max(1, std::min(device_slot
 int grad_slabs(mset_ctx* c) { return grad_slabs(c, c->ws->shape); }
 
 // The workgroup shape of a batched launch.  A launch with at most one position per CU takes the large workgroup
-// where the default one is sized for several positions per CU: with stored waves at 48 (201 -> 128 us at 256
+// where the default one is sized for several positions per CU: with stored waves at 48 (202 -> 150 us at 256
 // positions x 12 planes; from 400 on the default is faster, 220 against 248), and in the separable 256 routine
 // with stored or checkpointed waves (a tilt's last mini-batch, 15-20 % shorter at 64-256 positions).  The line
-// transforms, operand order and slab assignment are the default shape's, so the gradient slabs are the same up
-// to the compiler's contraction of products (bit for bit at 256); the workgroup sums (loss, position terms)
-// add their terms in another order.
-int batch_shape(const mset_ctx* c, int shape, bool sep, int waves, int count, bool fixed) {
+// transforms, operand order and slab assignment are the default shape's, so the gradient slabs are the same bit
+// for bit; the workgroup sums (loss, position terms) add their terms in another order.
+int batch_shape(const mset_ctx* c, int shape, bool sep, int waves, int count) {
     if (shape != 0 || count > c->cus) return shape;
-    if (c->n == 48 && waves == WAVES_STORE && !fixed) return 2;
+    if (c->n == 48 && waves == WAVES_STORE) return 2;
     return c->n == 256 && sep && (waves == WAVES_STORE || waves == WAVES_CHECKPOINT) ? 2 : 0;
 }
-// the same for the forward-only kernels (78 -> 62 us at 48 and up to 256 positions, 94 against 117 at 400)
+// the same for the forward-only kernels
 int fwd_shape(const mset_ctx* c, int count) { return c->n == 48 && count <= c->cus ? 2 : 0; }
 
 // grid of a batched launch of `count` positions on S slabs: at most `want` workgroups and, when slabs take
@@ -540,7 +540,7 @@ int issue_grad(mset_ctx* c, int first, int count, bool apply, int want) {
     {
         Timed t(c, "position_batch");
         if (W.shape == SHAPE_SEP) HIPCHK(launch_sep_batch(c->n, A, grid, c->stream));
-        else HIPCHK(launch_batch(c->n, A, grid, batch_shape(c, W.shape, sep, W.waves, count, !apply), c->stream));
+        else HIPCHK(launch_batch(c->n, A, grid, batch_shape(c, W.shape, sep, W.waves, count), c->stream));
     }
     HIPCHK(launch_reduce_slabs(W.gslab.p, used, (size_t)planes(c) * plane(c), W.G.p, c->stream));
     if (sep) HIPCHK(launch_untranspose_odd(W.G.p, c->n, c->L, c->stream));
@@ -970,7 +970,7 @@ int mset_grad_noalloc(mset_ctx* c, int first, int count, float* dV, float* dprob
     A.sep = sep ? 1 : 0;
     A.tph = (const float*)trans;
     A.tph_b = (const float*)trans + L * n2;
-    HIPCHK(launch_batch(c->n, A, G, batch_shape(c, shape, sep, WAVES_STORE, count, true), c->stream));
+    HIPCHK(launch_batch(c->n, A, G, batch_shape(c, shape, sep, WAVES_STORE, count), c->stream));
     HIPCHK(launch_reduce_slabs(gslab, S, L * n2, dV, c->stream));
     if (sep) HIPCHK(launch_untranspose_odd(dV, c->n, c->L, c->stream));
     HIPCHK(launch_reduce_cslabs(pslab, S, n2, pslab, c->stream));
@@ -992,7 +992,7 @@ int mset_waves(mset_ctx* c, int k, float* waves_out) {
     A.want = 0;
     A.waves = WAVES_STORE;
     A.nslab = 1;
-    HIPCHK(launch_batch(c->n, A, 1, c->n < 128 && c->n != 48 ? 1 : 0, c->stream));
+    HIPCHK(launch_batch(c->n, A, 1, 0, c->stream));
     HIPCHK(hipMemcpyAsync(waves_out, c->ws->save.p, sizeof(float2) * (size_t)(c->L + 1) * plane(c),
                           hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));

@@ -27,7 +27,6 @@
 // k < N, computed on the host in double precision.
 #pragma once
 #include <hip/hip_runtime.h>
-#include <utility>
 
 namespace mset {
 
@@ -271,49 +270,10 @@ template <int G, class Ld, class Ap, int PF, bool EG> struct PrefetchOf<Staged<G
 };
 
 // ------------------------------------------------------------------ one Stockham stage
-// Operands of a staged functor for the elements a thread holds in one stage (empty for other functors), loaded
-// together: loaded where each element is stored, they would be one memory latency per element, since a wait
-// for a load also waits for every older store.  Up to STAGE_REGS registers of operands are loaded for all of the
-// thread's butterflies before the stage's LDS reads, so that the stage hides their latency; more of them are
-// loaded one butterfly at a time ahead of its transform.
-constexpr int STAGE_REGS = 48;
-template <class F, int CNT, int R, bool ON> struct StageOps {
-    template <class PT> __device__ __forceinline__ void load(const F&, PT) {}
-    template <class PT> __device__ __forceinline__ void load(const F&, PT, int) {}
-    __device__ __forceinline__ float2 apply(const F& f, const Pt& p, float2 v, int, int) const { return f(p, v); }
-};
-template <class F, int CNT, int R> struct StageOps<F, CNT, R, true> {
-    using Op = decltype(std::declval<const F&>().load(Pt{}));
-    static constexpr bool BULK = CNT * R * (int)(sizeof(Op) / 4) <= STAGE_REGS;
-    Op op[BULK ? CNT : 1][R];
-    // at(c, r, p): whether the thread has element r of butterfly c, and its point
-    template <class PT> __device__ __forceinline__ void load1(const F& f, PT at, int c) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            Pt p;
-            if (at(c, r, p)) op[BULK ? c : 0][r] = f.load(p);
-        }
-    }
-    template <class PT> __device__ __forceinline__ void load(const F& f, PT at) {
-        if constexpr (BULK) {
-#pragma unroll
-            for (int c = 0; c < CNT; ++c) load1(f, at, c);
-        }
-    }
-    template <class PT> __device__ __forceinline__ void load(const F& f, PT at, int c) {
-        if constexpr (!BULK) load1(f, at, c);
-    }
-    __device__ __forceinline__ float2 apply(const F& f, const Pt& p, float2 v, int c, int r) const {
-        return f.apply(p, v, op[BULK ? c : 0][r]);
-    }
-};
-
 // ROWS: transform along x (lines are rows y); otherwise along y (lines are columns x).
 // NS: span (product of the radices already done).  FIRST: apply `pre` on load (LOADG: pre supplies the
 // value, LDS is not read).  LAST: apply `post` on store.
-// AHEAD: load staged operands together (StageOps); otherwise they are loaded element by element.
-template <int N, int NT, int R, int NS, bool INV, bool ROWS, bool FIRST, bool LOADG, bool LAST, bool AHEAD, class Pre,
-          class Post>
+template <int N, int NT, int R, int NS, bool INV, bool ROWS, bool FIRST, bool LOADG, bool LAST, class Pre, class Post>
 __device__ __forceinline__ void fft_stage(float2* __restrict__ s, const float2* __restrict__ tw, const Pre& pre,
                                           const Post& post) {
     constexpr int S = Pitch<N>::S;
@@ -322,48 +282,32 @@ __device__ __forceinline__ void fft_stage(float2* __restrict__ s, const float2* 
     constexpr int CNT = (NB + NT - 1) / NT;   // butterflies per thread
     constexpr int TWS = N / (NS * R);         // twiddle table stride
     const int t = threadIdx.x;
-    auto point = [&](int line, int e) {
-        const int y = ROWS ? line : e, x = ROWS ? e : line;
-        return Pt{y, x, Idx{(unsigned)(ROWS ? x * N + y : y * N + x), 0u}};
-    };
-    auto base = [&](int j) { return (j / NS) * NS * R + j % NS; };
-    StageOps<Pre, CNT, R, AHEAD && FIRST && IsStaged<Pre>::value> pre_op;
-    StageOps<Post, CNT, R, AHEAD && LAST && IsStaged<Post>::value> post_op;
-    auto at_pre = [&](int c, int r, Pt& p) {
-        const int b = t + c * NT;
-        p = point(b % N, b / N + r * NL);
-        return NB % NT == 0 || b < NB;
-    };
-    auto at_post = [&](int c, int r, Pt& p) {
-        const int b = t + c * NT;
-        p = point(b % N, base(b / N) + r * NS);
-        return NB % NT == 0 || b < NB;
-    };
-    pre_op.load(pre, at_pre);
-    post_op.load(post, at_post);
     float2 v[CNT][R];
 #pragma unroll
     for (int c = 0; c < CNT; ++c) {
         const int b = t + c * NT;
         if (NB % NT == 0 || b < NB) {
             const int line = b % N, j = b / N;
-            pre_op.load(pre, at_pre, c);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const Pt pt = point(line, j + r * NL);
-                if constexpr (FIRST) v[c][r] = pre_op.apply(pre, pt, LOADG ? make_float2(0.f, 0.f) : s[pt.y * S + pt.x], c, r);
-                else v[c][r] = s[pt.y * S + pt.x];
+                const int e = j + r * NL;
+                const int y = ROWS ? line : e, x = ROWS ? e : line;
+                float2 val;
+                const Pt pt{y, x, Idx{(unsigned)(ROWS ? x * N + y : y * N + x), 0u}};
+                if constexpr (FIRST && LOADG) val = pre(pt, make_float2(0.f, 0.f));
+                else if constexpr (FIRST) val = pre(pt, s[y * S + x]);
+                else val = s[y * S + x];
+                v[c][r] = val;
             }
         }
     }
-    if constexpr (!(AHEAD && FIRST && LOADG)) __syncthreads();   // LDS was read
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < CNT; ++c) {
         const int b = t + c * NT;
         if (NB % NT == 0 || b < NB) {
             const int line = b % N, j = b / N;
             const int k = j % NS;
-            post_op.load(post, at_post, c);
             if constexpr (NS > 1) {
 #pragma unroll
                 for (int r = 1; r < R; ++r) {
@@ -373,41 +317,43 @@ __device__ __forceinline__ void fft_stage(float2* __restrict__ s, const float2* 
                 }
             }
             DFT<R, INV>::run(v[c]);
+            const int base = (j / NS) * NS * R + k;
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const Pt pt = point(line, base(j) + r * NS);
+                const int e = base + r * NS;
+                const int y = ROWS ? line : e, x = ROWS ? e : line;
                 float2 val = v[c][r];
-                if constexpr (LAST) val = post_op.apply(post, pt, val, c, r);
-                s[pt.y * S + pt.x] = val;
+                if constexpr (LAST) val = post(Pt{y, x, Idx{(unsigned)(ROWS ? x * N + y : y * N + x), 0u}}, val);
+                s[y * S + x] = val;
             }
         }
     }
     __syncthreads();
 }
 
-template <int N, int NT, bool AHEAD, bool INV, bool ROWS, int ST, int NS, bool FIRSTPASS, bool LOADG, bool LASTPASS,
-          class Pre, class Post>
+template <int N, int NT, bool INV, bool ROWS, int ST, int NS, bool FIRSTPASS, bool LOADG, bool LASTPASS, class Pre,
+          class Post>
 __device__ __forceinline__ void fft_pass(float2* s, const float2* tw, const Pre& pre, const Post& post) {
     if constexpr (ST < Plan<N>::S) {
         constexpr int R = Plan<N>::R[ST];
-        fft_stage<N, NT, R, NS, INV, ROWS, FIRSTPASS && ST == 0, LOADG, LASTPASS && ST == Plan<N>::S - 1, AHEAD>(s, tw, pre,
-                                                                                                               post);
-        fft_pass<N, NT, AHEAD, INV, ROWS, ST + 1, NS * R, FIRSTPASS, LOADG, LASTPASS>(s, tw, pre, post);
+        fft_stage<N, NT, R, NS, INV, ROWS, FIRSTPASS && ST == 0, LOADG, LASTPASS && ST == Plan<N>::S - 1>(s, tw, pre,
+                                                                                                        post);
+        fft_pass<N, NT, INV, ROWS, ST + 1, NS * R, FIRSTPASS, LOADG, LASTPASS>(s, tw, pre, post);
     }
 }
 
 // Forward 2D transform: columns (pre fused, lanes along x) then rows (post fused, lanes along y).
-template <int N, int NT, bool AHEAD, bool LOADG = false, class Pre = NoOp, class Post = NoOp>
+template <int N, int NT, bool LOADG = false, class Pre = NoOp, class Post = NoOp>
 __device__ __forceinline__ void fft2d_fwd(float2* s, const float2* tw, const Pre& pre = Pre(), const Post& post = Post()) {
-    fft_pass<N, NT, AHEAD, false, false, 0, 1, true, LOADG, false>(s, tw, pre, post);
-    fft_pass<N, NT, AHEAD, false, true, 0, 1, false, false, true>(s, tw, pre, post);
+    fft_pass<N, NT, false, false, 0, 1, true, LOADG, false>(s, tw, pre, post);
+    fft_pass<N, NT, false, true, 0, 1, false, false, true>(s, tw, pre, post);
 }
 
 // Inverse 2D transform (no 1/N^2): rows (pre fused, lanes along y) then columns (post fused, lanes along x).
-template <int N, int NT, bool AHEAD, bool LOADG = false, class Pre = NoOp, class Post = NoOp>
+template <int N, int NT, bool LOADG = false, class Pre = NoOp, class Post = NoOp>
 __device__ __forceinline__ void fft2d_inv(float2* s, const float2* tw, const Pre& pre = Pre(), const Post& post = Post()) {
-    fft_pass<N, NT, AHEAD, true, true, 0, 1, true, LOADG, false>(s, tw, pre, post);
-    fft_pass<N, NT, AHEAD, true, false, 0, 1, false, false, true>(s, tw, pre, post);
+    fft_pass<N, NT, true, true, 0, 1, true, LOADG, false>(s, tw, pre, post);
+    fft_pass<N, NT, true, false, 0, 1, false, false, true>(s, tw, pre, post);
 }
 
 // ------------------------------------------------------------------ batched 1D transforms of a tile of lines
@@ -468,7 +414,7 @@ __device__ __forceinline__ void line_fft(float2* s, const float2* tw) {
 // The LDS-stage transforms behind the engine interface shared with the register-resident engine:
 // fwd / inv with (y, x, value) functors, each_R / each_C to visit the plane after a forward / inverse
 // transform (lanes along y, resp. along x, so [x][y] resp. [y][x] global arrays stay coalesced).
-template <int N, int NT_, bool AHEAD = false> struct LdsEngine {
+template <int N, int NT_> struct LdsEngine {
     static constexpr int NT = NT_;
     static constexpr int S = Pitch<N>::S;
     static constexpr int LDS_ELEMS = N * S;
@@ -483,11 +429,11 @@ template <int N, int NT_, bool AHEAD = false> struct LdsEngine {
     __device__ __forceinline__ void bind(float2*) {}   // the plane lives in LDS
     template <bool LOADG = false, class Pre = NoOp, class Post = NoOp>
     __device__ __forceinline__ void fwd(const Pre& pre = Pre(), const Post& post = Post()) {
-        fft2d_fwd<N, NT, AHEAD, LOADG>(s, tw, pre, post);
+        fft2d_fwd<N, NT, LOADG>(s, tw, pre, post);
     }
     template <bool LOADG = false, class Pre = NoOp, class Post = NoOp>
     __device__ __forceinline__ void inv(const Pre& pre = Pre(), const Post& post = Post()) {
-        fft2d_inv<N, NT, AHEAD, LOADG>(s, tw, pre, post);
+        fft2d_inv<N, NT, LOADG>(s, tw, pre, post);
     }
     template <class F> __device__ __forceinline__ void each_R(const F& f) {
         for (int i = threadIdx.x; i < N * N; i += NT) {

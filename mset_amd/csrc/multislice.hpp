@@ -42,31 +42,28 @@ namespace mset {
 // (HIP launch bounds).
 //
 // SH = 0: the shape of the batched and forward-only kernels.  Below 128 a position's time is the latency of its
-// chain of short LDS stages, so it takes enough threads for 4 to 12 elements each with the staged operands
-// loaded together ahead of the stage (AHEAD), rather than 9 to 18 elements with one load latency each.
-// Batched gradient of 256 / 1400 positions x 12 planes, 64 to 256 threads (576 at 96) against the shapes here:
-// 51 -> 44 / 68 -> 54 us at 16, 120 -> 70 / 157 -> 160 at 24, 211 -> 73 / 256 -> 170 at 32,
-// 301 -> 169 / 920 -> 780 at 64, and 726 -> 415 us for 256, 2108 -> 1229 for 700 positions at 96.  (At 64 a
-// budget of 4 waves per SIMD, two workgroups per CU, is 7 % slower at 256 positions and 14 % faster at 1400.)
-// At 48 the small workgroup is the better one once positions share a CU (654 against 721 us at 1400) and
-// the large one, SH = 2, below that (201 -> 128 us at 256).
+// chain of short LDS stages, so it takes enough threads for 4 to 12 elements each rather than 9 to 18, with the
+// same arithmetic and results.  Batched gradient of 256 / 1400 positions x 12 planes, with 64 threads (256 at 64, 576
+// at 96) against the shapes here: 119 -> 73 / 157 -> 157 us at 24, 171 -> 85 / 223 -> 190 at 32, 320 -> 204 /
+// 1001 -> 898 at 64, and 581 -> 443 us for 256, 1761 -> 1329 for 700 positions at 96.  (At 64 a budget of 4 waves per
+// SIMD, two workgroups per CU, is 5 % slower at 256 positions and 20 % faster at 1400.)  At 48 the small workgroup is
+// the better one once positions share a CU (665 against 721 us at 1400) and the large one, SH = 2, below that
+// (202 -> 150 us at 256).  These kernels serve what the on-chip separable routine (sep_lines.hpp) does not: mset_grad,
+// the exact pairing, recomputed and checkpointed waves, other propagators, the single-slice operator.
 // SH = 1: the alternative shape of the batched kernel, a candidate for the autotuner (MSET_ENGINE_ALT_SHAPE):
-// smaller workgroups with operands loaded element by element (at 48 a larger one); at 128 the register engine
-// with a half-size transpose buffer and a 128-register budget (two workgroups per CU instead of one; it spills
-// about 400 registers); tiles of 16 lines with 256 threads (three workgroups per CU instead of two) at 256.
-// Below 128 (other than 48) mset_grad runs this shape: the compiler contracts the products of the two differently
-// (2e-7 of the waves), which position terms that cancel turn into 1e-4 of a gradient, and gradients are
-// what callers difference.
+// smaller workgroups below 128 (at 48 a larger one); at 128 the register engine with a half-size transpose buffer
+// and a 128-register budget (two workgroups per CU instead of one; it spills about 400 registers); tiles of 16 lines
+// with 256 threads (three workgroups per CU instead of two) at 256.
 // SH = 2: launches of at most one position per CU and the one-position kernel: at 48 a workgroup of 768, at 256
 // 64-line tiles, one workgroup of 16 waves per CU with twice the default workgroup's loads in flight; the
 // default shape elsewhere.
 template <int N, int SH = 0> struct Cfg;
-template <> struct Cfg<16> { static constexpr int NT = 64, MINB = 1;  using Eng = LdsEngine<16, 64, true>; };
-template <> struct Cfg<24> { static constexpr int NT = 192, MINB = 1; using Eng = LdsEngine<24, 192, true>; };
-template <> struct Cfg<32> { static constexpr int NT = 256, MINB = 1; using Eng = LdsEngine<32, 256, true>; };
+template <> struct Cfg<16> { static constexpr int NT = 64, MINB = 1;  using Eng = LdsEngine<16, 64>; };
+template <> struct Cfg<24> { static constexpr int NT = 192, MINB = 1; using Eng = LdsEngine<24, 192>; };
+template <> struct Cfg<32> { static constexpr int NT = 256, MINB = 1; using Eng = LdsEngine<32, 256>; };
 template <> struct Cfg<48> { static constexpr int NT = 192, MINB = 1; using Eng = LdsEngine<48, 192>; };
-template <> struct Cfg<64> { static constexpr int NT = 512, MINB = 4; using Eng = LdsEngine<64, 512, true>; };
-template <> struct Cfg<96> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<96, 768, true>; };
+template <> struct Cfg<64> { static constexpr int NT = 512, MINB = 4; using Eng = LdsEngine<64, 512>; };
+template <> struct Cfg<96> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<96, 768>; };
 template <> struct Cfg<128> { static constexpr int NT = 512, MINB = 1; using Eng = RegEngine<128>; };
 template <> struct Cfg<256> { static constexpr int NT = 512, MINB = 4; using Eng = TiledEngine<256, 512>; };
 template <> struct Cfg<16, 1> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<16, 64>; };
@@ -75,10 +72,10 @@ template <> struct Cfg<32, 1> { static constexpr int NT = 64, MINB = 1; using En
 template <> struct Cfg<48, 1> { static constexpr int NT = 384, MINB = 1; using Eng = LdsEngine<48, 384>; };
 template <> struct Cfg<64, 1> { static constexpr int NT = 256, MINB = 3; using Eng = LdsEngine<64, 256>; };
 template <> struct Cfg<96, 1> { static constexpr int NT = 576, MINB = 1; using Eng = LdsEngine<96, 576>; };
-template <> struct Cfg<128, 1> { static constexpr int NT = 512, MINB = 4; using Eng = RegEngine<128, true>; };
+template <> struct Cfg<128, 1> { static constexpr int NT = 512, MINB = 4; using Eng = RegEngine<128>; };
 template <> struct Cfg<256, 1> { static constexpr int NT = 256, MINB = 3; using Eng = TiledEngine<256, 256>; };
 template <int N> struct Cfg<N, 2> : Cfg<N> {};
-template <> struct Cfg<48, 2> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<48, 768, true>; };
+template <> struct Cfg<48, 2> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<48, 768>; };
 template <> struct Cfg<256, 2> { static constexpr int NT = 1024, MINB = 4; using Eng = TiledEngine<256, 1024>; };
 
 
