@@ -48,22 +48,46 @@ __global__ void k_tv_scale(const float* __restrict__ f, long long nv, float lamb
         q[i] = f[i] / lambda;
 }
 
-// W consecutive elements of a row, one load or store
+// W consecutive elements of a row
 template <int W> struct Row {
     float a[W];
-    __device__ __forceinline__ static Row at(const float* p) {
-        Row r;
+};
+
+// One volume: a buffer view with 32-bit offsets (I = unsigned), or a pointer for volumes beyond its reach
+template <int W, class I> struct Volume {
+    float* p;
+    __device__ __forceinline__ Volume(const float* q, size_t) : p(const_cast<float*>(q)) {}
+    __device__ __forceinline__ float one(I i) const { return p[i]; }
+    __device__ __forceinline__ Row<W> row(I i) const {
+        Row<W> r;
         if constexpr (W == 4) {
-            const float4 t = *reinterpret_cast<const float4*>(p);
+            const float4 t = *reinterpret_cast<const float4*>(p + i);
             r.a[0] = t.x; r.a[1] = t.y; r.a[2] = t.z; r.a[3] = t.w;
         } else {
-            r.a[0] = *p;
+            r.a[0] = p[i];
         }
         return r;
     }
-    __device__ __forceinline__ void put(float* p) const {
-        if constexpr (W == 4) *reinterpret_cast<float4*>(p) = make_float4(a[0], a[1], a[2], a[3]);
-        else *p = a[0];
+    __device__ __forceinline__ void put(I i, const Row<W>& r) const {
+        if constexpr (W == 4) *reinterpret_cast<float4*>(p + i) = make_float4(r.a[0], r.a[1], r.a[2], r.a[3]);
+        else p[i] = r.a[0];
+    }
+};
+template <int W> struct Volume<W, unsigned> {
+    typedef unsigned u32x4 __attribute__((__vector_size__(16)));
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ Volume(const float* q, size_t n)
+        : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(q), (short)0, (int)(unsigned)(n * 4), 0x00020000)) {}
+    __device__ __forceinline__ float one(unsigned i) const {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, i * 4u, 0, 0));
+    }
+    __device__ __forceinline__ Row<W> row(unsigned i) const {
+        if constexpr (W == 4) return __builtin_bit_cast(Row<4>, __builtin_amdgcn_raw_buffer_load_b128(r, i * 4u, 0, 0));
+        else return Row<1>{one(i)};
+    }
+    __device__ __forceinline__ void put(unsigned i, const Row<W>& v) const {
+        if constexpr (W == 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, i * 4u, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v.a[0]), r, i * 4u, 0, 0);
     }
 };
 
@@ -71,44 +95,43 @@ template <int W> struct Row {
 // and of their x, y and z successors is formed from P (25 loads for 4 elements, all but 7 of them hits in
 // L1 or L2, requested together), so D is never stored and P, q are read once and P written once: 28 bytes of
 // memory traffic per element instead of 48 in two launches with a stored D.  q = f / lambda is formed once.  The
-// fields alternate between Pi and Po.  64 x 128 x 128 volume: 13.8 us per iteration as two launches with 64-bit
-// index divisions, 8.3 us now, bound by the 29 MB that a launch reads from and writes back past L2.
-// I: index type, 32-bit unless the volume needs more (64-bit divisions cost more than the stencil).
+// fields alternate between Pi and Po.  A neighbour is the element's index plus a step that wraps at the volume's
+// faces, in 32 bits (I) unless the volume needs more: index arithmetic in 64 bits took a third of the kernel's
+// instructions.  64 x 128 x 128 volume, per iteration: 13.8 us as two launches, 8.3 us with pointers, 7.8 us with
+// views.
 template <int W, class I>
 __global__ __launch_bounds__(256) void k_tv_iterate(int nx, int ny, int nz, const float* __restrict__ Pi,
-                                                    const float* __restrict__ q, float* __restrict__ Po, I items) {
+                                                    const float* __restrict__ q_, float* __restrict__ Po, I items) {
     const float tau = 1.0f / 12.0f;
-    const size_t nv = (size_t)nx * ny * nz, sz = (size_t)nx * ny;
-    const float *P0 = Pi, *P1 = Pi + nv, *P2 = Pi + 2 * nv;
+    const size_t nv = (size_t)nx * ny * nz;
+    using Vol = Volume<W, I>;
+    using V = Row<W>;
+    const Vol P0(Pi, nv), P1(Pi + nv, nv), P2(Pi + 2 * nv, nv), q(q_, nv);
+    const Vol O0(Po, nv), O1(Po + nv, nv), O2(Po + 2 * nv, nv);
     const unsigned rows = (unsigned)nx / W;
+    const I row = (I)nx, plane = (I)nx * (I)ny, depth = plane * (I)nz;
     // Workgroups go to the 8 XCDs round-robin: renumbered so that each XCD works on one contiguous part of the
     // volume and finds the neighbouring rows and planes in its own L2
     const unsigned g = gridDim.x, b = g % 8 == 0 ? blockIdx.x % 8 * (g / 8) + blockIdx.x / 8 : blockIdx.x;
     for (I i = (I)b * blockDim.x + threadIdx.x; i < items; i += (I)g * blockDim.x) {
-        const unsigned x = (unsigned)(i % rows) * W;
-        const I yz = i / rows;
-        const unsigned y = (unsigned)(yz % (unsigned)ny), z = (unsigned)(yz / (unsigned)ny);
-        // rows at (y, z) and its neighbours, periodic
-        const unsigned yp = y + 1 == (unsigned)ny ? 0 : y + 1, ym = y == 0 ? ny - 1 : y - 1;
-        const unsigned zp = z + 1 == (unsigned)nz ? 0 : z + 1, zm = z == 0 ? nz - 1 : z - 1;
-        const unsigned xm = x == 0 ? nx - 1 : x - 1, xp = x + W == (unsigned)nx ? 0 : x + W;
-        const size_t r = z * sz + (size_t)y * nx, ryp = z * sz + (size_t)yp * nx, rym = z * sz + (size_t)ym * nx;
-        const size_t rzp = zp * sz + (size_t)y * nx, rzm = zm * sz + (size_t)y * nx;
-        const size_t rypzm = zm * sz + (size_t)yp * nx, rzpym = zp * sz + (size_t)ym * nx;
-        using V = Row<W>;
-        const V a = V::at(P0 + r + x), b = V::at(P1 + r + x), c = V::at(P2 + r + x);
-        const V bym = V::at(P1 + rym + x), czm = V::at(P2 + rzm + x), f = V::at(q + r + x);
-        const float am = P0[r + xm];
+        const I e = i * W, yz = i / rows, z = yz / (unsigned)ny;
+        const unsigned x = (unsigned)(i - yz * rows) * W, y = (unsigned)(yz - z * (unsigned)ny);
+        // neighbours, periodic (unsigned differences wrap around to the right index)
+        const I xp = (x + W == (unsigned)nx ? (I)W - row : (I)W), xm = x == 0 ? row - 1 : (I)0 - 1;
+        const I yp = y + 1 == (unsigned)ny ? row - plane : row, ym = y == 0 ? plane - row : (I)0 - row;
+        const I zp = z + 1 == (I)nz ? plane - depth : plane, zm = z == 0 ? depth - plane : (I)0 - plane;
+        const V a = P0.row(e), b_ = P1.row(e), c = P2.row(e);
+        const V bym = P1.row(e + ym), czm = P2.row(e + zm), f = q.row(e);
+        const float am = P0.one(e + xm);
         // x successor of the last element
-        const float ax = P0[r + xp], bx = P1[r + xp], cx = P2[r + xp], bxym = P1[rym + xp], cxzm = P2[rzm + xp], fx = q[r + xp];
+        const float ax = P0.one(e + xp), bx = P1.one(e + xp), cx = P2.one(e + xp), bxym = P1.one(e + xp + ym);
+        const float cxzm = P2.one(e + xp + zm), fx = q.one(e + xp);
         // y successors
-        const V ay = V::at(P0 + ryp + x), by = V::at(P1 + ryp + x), cy = V::at(P2 + ryp + x);
-        const V cyzm = V::at(P2 + rypzm + x), fy = V::at(q + ryp + x);
-        const float aym = P0[ryp + xm];
+        const V ay = P0.row(e + yp), by = P1.row(e + yp), cy = P2.row(e + yp), cyzm = P2.row(e + yp + zm), fy = q.row(e + yp);
+        const float aym = P0.one(e + yp + xm);
         // z successors
-        const V az = V::at(P0 + rzp + x), bz = V::at(P1 + rzp + x), cz = V::at(P2 + rzp + x);
-        const V bzym = V::at(P1 + rzpym + x), fz = V::at(q + rzp + x);
-        const float azm = P0[rzp + xm];
+        const V az = P0.row(e + zp), bz = P1.row(e + zp), cz = P2.row(e + zp), bzym = P1.row(e + zp + ym), fz = q.row(e + zp);
+        const float azm = P0.one(e + zp + xm);
         // TV_div in its operation order, then - f / lambda
         auto res = [](float p0, float p1, float p2, float p0m, float p1m, float p2m, float g) {
             float d = p0 + p1 + p2;
@@ -119,15 +142,15 @@ __global__ __launch_bounds__(256) void k_tv_iterate(int nx, int ny, int nz, cons
         };
         float d[W + 1];
 #pragma unroll
-        for (int k = 0; k < W; ++k) d[k] = res(a.a[k], b.a[k], c.a[k], k ? a.a[k - 1] : am, bym.a[k], czm.a[k], f.a[k]);
+        for (int k = 0; k < W; ++k) d[k] = res(a.a[k], b_.a[k], c.a[k], k ? a.a[k - 1] : am, bym.a[k], czm.a[k], f.a[k]);
         d[W] = res(ax, bx, cx, a.a[W - 1], bxym, cxzm, fx);
         V o0, o1, o2;
 #pragma unroll
         for (int k = 0; k < W; ++k) {
-            const float dy = res(ay.a[k], by.a[k], cy.a[k], k ? ay.a[k - 1] : aym, b.a[k], cyzm.a[k], fy.a[k]);
+            const float dy = res(ay.a[k], by.a[k], cy.a[k], k ? ay.a[k - 1] : aym, b_.a[k], cyzm.a[k], fy.a[k]);
             const float dz = res(az.a[k], bz.a[k], cz.a[k], k ? az.a[k - 1] : azm, bzym.a[k], c.a[k], fz.a[k]);
             const float q0 = a.a[k] + tau * (d[k + 1] - d[k]);
-            const float q1 = b.a[k] + tau * (dy - d[k]);
+            const float q1 = b_.a[k] + tau * (dy - d[k]);
             const float q2 = c.a[k] + tau * (dz - d[k]);
             // den = sqrt(max(1, |q|^2)) and the three quotients with it, each the hardware's estimate corrected by
             // its remainder (Markstein, IBM J. Res. Dev. 34 (1990) 111): the arguments are normal and near 1, so the
@@ -145,9 +168,9 @@ __global__ __launch_bounds__(256) void k_tv_iterate(int nx, int ny, int nz, cons
             o1.a[k] = quot(q1);
             o2.a[k] = quot(q2);
         }
-        o0.put(Po + r + x);
-        o1.put(Po + nv + r + x);
-        o2.put(Po + 2 * nv + r + x);
+        O0.put(e, o0);
+        O1.put(e, o1);
+        O2.put(e, o2);
     }
 }
 
@@ -249,7 +272,7 @@ hipError_t tv_run(TvWork& w, const float* f, float* u, int nx, int ny, int nz, f
     hipLaunchKernelGGL(k_tv_scale, gr, bl, 0, st, f, nv, lambda, q);
     const bool wide = nx % 4 == 0;                       // rows of whole float4s
     const long long items = wide ? nv / 4 : nv;
-    const bool narrow_index = items < (1LL << 31);
+    const bool narrow_index = nv < (1LL << 30);          // 32-bit byte offsets
     for (int it = 0; it < n_iter; ++it) {
         const dim3 gi = grid_of(items);
         if (wide && narrow_index)
