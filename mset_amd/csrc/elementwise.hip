@@ -3,6 +3,7 @@
 // accesses where the layout allows; launches are sized to the element count (>= 1024 workgroups when
 // the data is large) so the 256 CUs / 8 XCDs are filled.
 #include <hip/hip_runtime.h>
+#include <type_traits>
 #include "kernels.hpp"
 
 namespace mset {
@@ -104,34 +105,33 @@ __global__ void k_fill_bytes(unsigned char* p, size_t n) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0;
 }
 
-// out[i] = sum_s slab[s][i], s ascending (fixed order: bitwise repeatable)
-// Slabs are summed in slot order (s = 0, 1, ...), so the result is the same for every launch shape;
-// U loads are in flight at a time.
-__global__ void k_reduce(const float4* __restrict__ slab, int nslab, size_t n4, float4* __restrict__ out) {
-    constexpr int U = 8;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
-        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-        int s = 0;
-        for (; s + U <= nslab; s += U) {
-            float4 v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = slab[(size_t)(s + u) * n4 + i];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                a.x += v[u].x; a.y += v[u].y; a.z += v[u].z; a.w += v[u].w;
-            }
-        }
-        for (; s < nslab; ++s) {
-            const float4 v = slab[(size_t)s * n4 + i];
-            a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
-        }
-        out[i] = a;
-    }
+__device__ __forceinline__ void add_to(float& a, float b) { a += b; }
+__device__ __forceinline__ void add_to(float4& a, const float4& b) {
+    a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
 }
-__global__ void k_reduce1(const float* __restrict__ slab, int nslab, size_t n, float* __restrict__ out) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        float a = 0.f;
-        for (int s = 0; s < nslab; ++s) a += slab[(size_t)s * n + i];
+
+// out[i] = sum_s slab[s][i].  Slabs are summed in slot order (s = 0, 1, ...), so the result is the same for every
+// launch shape, and out may be slab 0 (an element is read and written by the same thread); U loads are in flight at
+// a time.  Bound by memory where the sum is large (5.2 TB/s for 256 slabs of 2^18 floats); a small one is a chain of
+// nslab / U memory latencies on few wavefronts, and takes one float per thread and U = 32.
+template <class T, int U>
+__global__ __launch_bounds__(256) void k_reduce(const T* slab, int nslab, size_t n, T* out) {
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        T a{};
+        int s = 0;
+        auto add = [&](auto count) {
+            constexpr int C = decltype(count)::value;
+            for (; s + C <= nslab; s += C) {
+                T v[C];
+#pragma unroll
+                for (int u = 0; u < C; ++u) v[u] = slab[(size_t)(s + u) * n + i];
+#pragma unroll
+                for (int u = 0; u < C; ++u) add_to(a, v[u]);
+            }
+        };
+        add(std::integral_constant<int, U>{});
+        if constexpr (U > 8) add(std::integral_constant<int, 8>{});
+        add(std::integral_constant<int, 1>{});
         out[i] = a;
     }
 }
@@ -188,10 +188,13 @@ hipError_t launch_fill(void* p, size_t bytes, hipStream_t st) {
 }
 
 hipError_t launch_reduce_slabs(const float* slab, int nslab, size_t n, float* out, hipStream_t st) {
-    if (n % 4 == 0 && ((uintptr_t)slab % 16) == 0 && ((uintptr_t)out % 16) == 0)
-        hipLaunchKernelGGL(k_reduce, grid_for(n / 4), dim3(256), 0, st, (const float4*)slab, nslab, n / 4, (float4*)out);
+    // float4 fills the chip from 2^16 floats on.  By 256 and 32 loads in flight: 2 x 96^2 floats in 200 slabs
+    // 13.4 -> 6.6 us, 2 x 128^2 in 256 slabs 15.2 -> 7.2; 12 x 96^2 in 200 slabs 16.4 (float4) against 17.2.
+    if (n > (size_t)1 << 16 && n % 4 == 0 && ((uintptr_t)slab % 16) == 0 && ((uintptr_t)out % 16) == 0)
+        hipLaunchKernelGGL((k_reduce<float4, 8>), grid_for(n / 4), dim3(256), 0, st, (const float4*)slab, nslab, n / 4,
+                           (float4*)out);
     else
-        hipLaunchKernelGGL(k_reduce1, grid_for(n), dim3(256), 0, st, slab, nslab, n, out);
+        hipLaunchKernelGGL((k_reduce<float, 32>), grid_for(n), dim3(256), 0, st, slab, nslab, n, out);
     return hipGetLastError();
 }
 
