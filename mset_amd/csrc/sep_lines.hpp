@@ -67,73 +67,71 @@ template <int N> struct SepLines {
         line = threadIdx.x / T;
         j = threadIdx.x % T;
 #pragma unroll
-        for (int k = 1; k < R1; ++k) w[k - 1] = tw[(j * k) % N];
+        for (int k = 1; k < R1; ++k) w[k - 1] = tw[jd() * k % N];
     }
     // Addresses are affine in (line, j); left visible, the compiler hoists them all out of the plane loops and keeps
     // a hundred registers live (see RegEngine::opaque)
     __device__ __forceinline__ void opaque() { asm volatile("" : "+v"(line), "+v"(j)); }
-    __device__ __forceinline__ bool in_d() const { return R2 == T || j < R2; }
-    __device__ __forceinline__ bool in_x(int c) const { return (c + 1) * T <= R1 || j + c * T < R1; }
-    // point of register i in layout X
-    __device__ __forceinline__ int xpos(int i) const { return j + (i / R2) * T + R1 * (i % R2); }
+    // Where a layout has fewer places than lanes (j >= R2 in D, j + c T >= R1 in X), the lanes beyond the last place
+    // duplicate it: same point, same values, same addresses written, so no access needs a mask or a branch.  Sums over
+    // the points leave them out (own_x, own_d).
+    __device__ __forceinline__ int jd() const { return R2 == T ? j : min(j, R2 - 1); }
+    __device__ __forceinline__ int jx(int c) const { return (c + 1) * T <= R1 ? j + c * T : min(j + c * T, R1 - 1); }
+    __device__ __forceinline__ bool own_d() const { return R2 == T || j < R2; }
+    __device__ __forceinline__ bool own_x(int i) const { return (i / R2 + 1) * T <= R1 || j + i / R2 * T < R1; }
 
     __device__ __forceinline__ void fwd() {
         opaque();
-        float2* ex = lds + line * LS;                       // this line's exchange slots
+        float2* ex = lds + __mul24(line, LS);               // this line's exchange slots
         DFT<R1, false>::run(v);
 #pragma unroll
         for (int k = 1; k < R1; ++k) v[k] = cmul(v[k], w[k - 1]);
-        if (in_d()) {
 #pragma unroll
-            for (int k = 0; k < R1; ++k) ex[k * EXP + j] = v[k];
-        }
+        for (int k = 0; k < R1; ++k) ex[jd() + k * EXP] = v[k];
         wave_lds_fence();
 #pragma unroll
-        for (int c = 0; c < CX; ++c)
-            if (in_x(c)) {
+        for (int c = 0; c < CX; ++c) {
+            const float2* q = ex + __mul24(jx(c), EXP);
 #pragma unroll
-                for (int i = 0; i < R2; ++i) v[c * R2 + i] = ex[(j + c * T) * EXP + i];
-            }
+            for (int i = 0; i < R2; ++i) v[c * R2 + i] = q[i];
+        }
         wave_lds_fence();
 #pragma unroll
         for (int c = 0; c < CX; ++c) DFT<R2, false>::run(v + c * R2);
     }
     __device__ __forceinline__ void inv() {
         opaque();
-        float2* ex = lds + line * LS;
+        float2* ex = lds + __mul24(line, LS);
 #pragma unroll
         for (int c = 0; c < CX; ++c) DFT<R2, true>::run(v + c * R2);
 #pragma unroll
-        for (int c = 0; c < CX; ++c)
-            if (in_x(c)) {
+        for (int c = 0; c < CX; ++c) {
+            float2* q = ex + __mul24(jx(c), EXP);
 #pragma unroll
-                for (int i = 0; i < R2; ++i) ex[(j + c * T) * EXP + i] = v[c * R2 + i];
-            }
-        wave_lds_fence();
-        if (in_d()) {
-#pragma unroll
-            for (int k = 0; k < R1; ++k) v[k] = ex[k * EXP + j];
+            for (int i = 0; i < R2; ++i) q[i] = v[c * R2 + i];
         }
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < R1; ++k) v[k] = ex[jd() + k * EXP];
         wave_lds_fence();
 #pragma unroll
         for (int k = 1; k < R1; ++k) v[k] = cmulc(v[k], w[k - 1]);
         DFT<R1, true>::run(v);
     }
 
-    // the points of layout D / X: f(register, point along the line)
+    // the points of layout D / X: f(register, lane's part of the point, the register's part)
     template <class F> __device__ __forceinline__ void each_d(const F& f) const {
-        if (in_d()) {
+        const int p = jd();
 #pragma unroll
-            for (int r = 0; r < R1; ++r) f(r, j + R2 * r);
-        }
+        for (int r = 0; r < R1; ++r) f(r, p, R2 * r);
     }
     template <class F> __device__ __forceinline__ void each_x(const F& f) const {
 #pragma unroll
-        for (int c = 0; c < CX; ++c)
-            if (in_x(c)) {
+        for (int c = 0; c < CX; ++c) {
+            const int p = jx(c);
 #pragma unroll
-                for (int i = 0; i < R2; ++i) f(c * R2 + i, xpos(c * R2 + i));
-            }
+            for (int i = 0; i < R2; ++i) f(c * R2 + i, p, R1 * i);
+        }
     }
     // turns the plane over: layout D or X of lines along one axis -> layout D or X of lines along the other.
     // col: the lines written are columns x (points y).
@@ -142,11 +140,11 @@ template <int N> struct SepLines {
         opaque();
         float2* pl = lds + (APART ? EX_ELEMS : 0);
         const int wl = col ? 1 : PITCH, wp = col ? PITCH : 1;
-        auto put = [&](int i, int pos) { pl[line * wl + pos * wp] = v[i]; };
+        auto put = [&](int i, int p, int q) { (pl + __mul24(line, wl) + __mul24(p, wp))[q * wp] = v[i]; };
         if constexpr (FROM_X) each_x(put);
         else each_d(put);
         __syncthreads();
-        auto get = [&](int i, int pos) { v[i] = pl[line * wp + pos * wl]; };
+        auto get = [&](int i, int p, int q) { v[i] = (pl + __mul24(line, wp) + __mul24(p, wl))[q * wl]; };
         if constexpr (TO_X) each_x(get);
         else each_d(get);
         if constexpr (!APART) __syncthreads();               // before exchanges write the shared slots
@@ -163,7 +161,7 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
     constexpr int N2 = N * N, R1 = Eng::R1, R2 = Eng::R2, EM = Eng::EM, NT = Eng::NT;
     constexpr bool GRAD = KIND != K_FWD;
     const int t = threadIdx.x, L = A.L;
-    const float inv_n = 1.0f / (float)N, inv_n2 = 1.0f / (float)N2;
+    const float inv_n2 = 1.0f / (float)N2;
     float2* save = A.save + (size_t)slot * (L + 2) * N2;
     const bool want_pos = GRAD && (A.want & WANT_POS) != 0;
     const bool want_probe = GRAD && (A.want & WANT_PROBE) != 0;
@@ -180,32 +178,33 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
     }
     __syncthreads();
 
-    // index of a point in a row-major [y][x] array (rm) and in a transposed [x][y] one (tm): the lane's part and, for
-    // layout D, the scalar part of register r
-    auto rm = [&](bool col, int pos) { return col ? pos * N + E.line : E.line * N + pos; };
-    auto tm = [&](bool col, int pos) { return col ? E.line * N + pos : pos * N + E.line; };
-    auto rm_d = [&](bool col, int r) {
-        return Idx{(unsigned)rm(col, E.j), (unsigned)(r * R2 * (col ? N : 1))};
+    // index of point p + q of the line in a row-major [y][x] array (rm) and in a transposed [x][y] one (tm): the lane's
+    // part and the register's (a constant for each orientation)
+    auto rm = [&](bool col, int p, int q) {
+        return Idx{(unsigned)(__mul24(E.line, col ? 1 : N) + __mul24(p, col ? N : 1)), (unsigned)(q * (col ? N : 1))};
     };
-    // propagation half-step factors along the pass axis (with the 1/N of its inverse transform)
+    auto tm = [&](bool col, int p, int q) { return rm(!col, p, q); };
+    auto rm_d = [&](bool col, int r) { return rm(col, E.jd(), r * R2); };
+    // propagation half-step factors along the pass axis (px, py hold the 1/N of its inverse transform)
     auto times_p = [&](bool col, bool conj) {
-        const float2* q = col ? py : px;
-        E.each_x([&](int i, int pos) {
-            const float2 f = q[pos];
-            E.v[i] = cscale(conj ? cmulc(E.v[i], f) : cmul(E.v[i], f), inv_n);
-        });
+        const float2* f = col ? py : px;
+        E.each_x([&](int i, int p, int q) { E.v[i] = conj ? cmulc(E.v[i], (f + p)[q]) : cmul(E.v[i], (f + p)[q]); });
     };
-    auto phase = [&](bool col, int pos) { return cmul(col ? phy[pos] : phy[E.line], col ? phx[E.line] : phx[pos]); };
+    auto phase = [&](bool col, int p, int q) {
+        return cmul(col ? (phy + p)[q] : phy[E.line], col ? phx[E.line] : (phx + p)[q]);
+    };
+    const BufC probe(KIND == K_PLAIN ? A.probe : const_cast<float2*>(A.probeF), N2);
+    const BufF MT(A.sqrtM + (size_t)k * N2, N2);             // [x][y]
 
     // ---- X0 (columns): fftn(probe) .* Phi, inverse along y
     if constexpr (KIND == K_PLAIN) {
-        E.each_d([&](int i, int pos) { E.v[i] = A.probe[rm(false, pos)]; });
+        E.each_d([&](int i, int p, int q) { E.v[i] = probe[rm(false, p, q)]; });
         E.fwd();
         E.template turn<true, false>(false);
         E.fwd();
-        E.each_x([&](int i, int pos) { E.v[i] = cmul(E.v[i], phase(true, pos)); });
+        E.each_x([&](int i, int p, int q) { E.v[i] = cmul(E.v[i], phase(true, p, q)); });
     } else {
-        E.each_x([&](int i, int pos) { E.v[i] = cmul(A.probeF[tm(true, pos)], phase(true, pos)); });
+        E.each_x([&](int i, int p, int q) { E.v[i] = cmul(probe[tm(true, p, q)], phase(true, p, q)); });
     }
     E.inv();
     E.template turn<false, true>(true);
@@ -224,7 +223,7 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
     {
         const BufC sv(save, N2);
         E.inv();
-        E.each_d([&](int r, int) {
+        E.each_d([&](int r, int, int) {
             const float2 u = cscale(E.v[r], inv_n2);
             if (GRAD) sv.put(rm_d(false, r), u);
             E.v[r] = cmul(u, o[r]);
@@ -236,14 +235,13 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
         E.template turn<false, false>(false);
     }
     // ---- X_(a+1): finish plane a-1's step, keep psi_a, x t_a, start plane a's step
-    for (int a = 1; a < L; ++a) {
-        const bool col = a & 1;
+    auto plane_fwd = [&](bool col, int a) __attribute__((always_inline)) {
         const BufC sv(save + (size_t)a * N2, N2);
         if (!EARLY) want_t(col, a);
         E.fwd();
         times_p(col, false);
         E.inv();
-        E.each_d([&](int r, int) {
+        E.each_d([&](int r, int, int) {
             if (GRAD) sv.put(rm_d(col, r), E.v[r]);
             E.v[r] = cmul(E.v[r], o[r]);
         });
@@ -252,18 +250,22 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
         times_p(col, false);
         E.inv();
         E.template turn<false, false>(col);
+    };
+    // a pass of each orientation: strides and offsets are constants
+    for (int a = 1; a < L; a += 2) {
+        plane_fwd(true, a);
+        if (a + 1 < L) plane_fwd(false, a + 1);
     }
     // ---- X_(L+1): finish plane L-1's step, keep psi_L, forward along this axis
     float m[EM];
-    const float* MT = A.sqrtM + (size_t)k * N2;              // [x][y]
     {
         const bool col = L & 1;
         const BufC sv(save + (size_t)L * N2, N2);
-        if (EARLY) E.each_x([&](int i, int pos) { m[i] = MT[tm(!col, pos)]; });
+        if (EARLY) E.each_x([&](int i, int p, int q) { m[i] = MT[tm(!col, p, q)]; });
         E.fwd();
         times_p(col, false);
         E.inv();
-        if (GRAD) E.each_d([&](int r, int) { sv.put(rm_d(col, r), E.v[r]); });
+        if (GRAD) E.each_d([&](int r, int, int) { sv.put(rm_d(col, r), E.v[r]); });
         E.fwd();
         E.template turn<true, false>(col);
     }
@@ -273,15 +275,15 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
     {
         const bool col = !(L & 1);
         float* Iout = A.inten ? A.inten + (size_t)k * N2 : nullptr;
-        if (!EARLY) E.each_x([&](int i, int pos) { m[i] = MT[tm(col, pos)]; });
+        if (!EARLY) E.each_x([&](int i, int p, int q) { m[i] = MT[tm(col, p, q)]; });
         E.fwd();
-        E.each_x([&](int i, int pos) {
+        E.each_x([&](int i, int p, int q) {
             const float2 u = E.v[i];
             const float I = u.x * u.x + u.y * u.y;
-            const int y = col ? pos : E.line, x = col ? E.line : pos;
+            const int y = col ? p + q : E.line, x = col ? E.line : p + q;
             if (KIND == K_FWD && Iout) Iout[((y + N / 2) % N) * N + (x + N / 2) % N] = I;
             const float d = m[i] - __builtin_amdgcn_sqrtf(I);
-            err += (double)(d * d);
+            if (E.own_x(i)) err += (double)(d * d);
             if constexpr (GRAD) {
                 const float f = 1.0f - m[i] * __builtin_amdgcn_rsqf(I + 1e-30f);
                 E.v[i] = cmulc(make_float2(u.x * f, u.y * f), cmul(px[x], py[y]));
@@ -300,8 +302,8 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
     double dr = 0.0, dc = 0.0;
     float2 wv[R1];
     float gi[R1];
-    for (int a = L - 1; a >= 0; --a) {
-        const bool col = !(a & 1), head = a == L - 1;
+    auto plane_back = [&](bool col, int a) __attribute__((always_inline)) {
+        const bool head = a == L - 1;
         const BufC ws(save + (size_t)(a + 1) * N2, N2);
         const BufF g(A.gslab + ((size_t)slab * L + a) * N2, N2);
         const BufF gin(A.gslab + ((size_t)slab * L + a) * N2, first ? 0u : N2);   // empty view: reads 0
@@ -316,8 +318,8 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
             times_p(col, true);
         }
         E.inv();
-        E.each_d([&](int r, int) {
-            const float2 u = head ? cscale(E.v[r], inv_n2) : E.v[r];
+        E.each_d([&](int r, int, int) {
+            const float2 u = E.v[r];
             const float2 tc = cconj(o[r]);
             const float gr = -cmul(tc, cmulc(u, wv[r])).y;   // Re(1i * conj(t) * conj(psi) * b)
             g.put(rm_d(col, r), KIND == K_BATCH ? gi[r] + gr : gr);
@@ -326,11 +328,12 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
         if (a == 0 && want_pos) {
             // position terms (STEP03_BACK.m:35-38): MATLAB gradient() of conj(psi0)
             const float2* p0 = save;
-            E.each_d([&](int r, int y) {
-                const int x = E.line;
+            E.each_d([&](int r, int p, int q) {
+                const int x = E.line, y = p + q;
                 const int xp = min(x + 1, N - 1), xm = max(x - 1, 0), yp = min(y + 1, N - 1), ym = max(y - 1, 0);
                 const float2 gx = cscale(csub(p0[y * N + xp], p0[y * N + xm]), xp - xm == 2 ? 0.5f : 1.0f);
                 const float2 gy = cscale(csub(p0[yp * N + x], p0[ym * N + x]), yp - ym == 2 ? 0.5f : 1.0f);
+                if (!E.own_d()) return;
                 dr += (double)(gx.x * E.v[r].x + gx.y * E.v[r].y);
                 dc += (double)(gy.x * E.v[r].x + gy.y * E.v[r].y);
             });
@@ -341,6 +344,10 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
             E.inv();
             E.template turn<false, false>(col);
         }
+    };
+    for (int a = (L - 1) | 1; a > 0; a -= 2) {
+        if (a < L) plane_back(false, a);
+        plane_back(true, a - 1);
     }
     if (want_pos) {
         dr = block_sum<NT>(dr, red);
@@ -359,22 +366,22 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
     if (want_probe) {
         E.template turn<true, false>(true);
         if constexpr (KIND == K_BATCH) {
-            const float2* in = A.pslab + (size_t)slab * N2;
-            float2* out = A.pslab + (size_t)slab * N2;
+            const BufC out(A.pslab + (size_t)slab * N2, N2);
+            const BufC in(A.pslab + (size_t)slab * N2, first ? 0u : N2);
             float2 o[EM];
-            E.each_x([&](int i, int pos) { o[i] = first ? make_float2(0.f, 0.f) : in[tm(false, pos)]; });
+            E.each_x([&](int i, int p, int q) { o[i] = in[tm(false, p, q)]; });
             E.fwd();
-            E.each_x([&](int i, int pos) { out[tm(false, pos)] = cadd(o[i], cmulc(E.v[i], phase(false, pos))); });
+            E.each_x([&](int i, int p, int q) { out.put(tm(false, p, q), cadd(o[i], cmulc(E.v[i], phase(false, p, q)))); });
         } else {
             E.fwd();
-            E.each_x([&](int i, int pos) { E.v[i] = cmulc(E.v[i], phase(false, pos)); });
+            E.each_x([&](int i, int p, int q) { E.v[i] = cmulc(E.v[i], phase(false, p, q)); });
             E.inv();
             E.template turn<false, true>(false);
             float2 o[R1];
-            E.each_d([&](int r, int pos) { o[r] = A.probe[rm(true, pos)]; });
+            E.each_d([&](int r, int p, int q) { o[r] = probe[rm(true, p, q)]; });
             E.inv();
-            E.each_d([&](int r, int pos) {
-                A.probe[rm(true, pos)] = csub(o[r], cscale(cscale(E.v[r], inv_n2), A.s2));
+            E.each_d([&](int r, int p, int q) {
+                probe.put(rm(true, p, q), csub(o[r], cscale(cscale(E.v[r], inv_n2), A.s2)));
             });
         }
     }
@@ -396,7 +403,7 @@ template <int N> struct SepCfg {
     __shared__ float2 s[Eng::LDS_ELEMS];                                        \
     __shared__ float2 phx[N], phy[N], px[N], py[N];                             \
     __shared__ double red[(NT + 63) / 64];                                      \
-    for (int i = threadIdx.x; i < 2 * N; i += NT) (i < N ? px : py)[i % N] = A.p1d[i]; \
+    for (int i = threadIdx.x; i < 2 * N; i += NT) (i < N ? px : py)[i % N] = cscale(A.p1d[i], 1.0f / N); \
     __syncthreads();                                                            \
     Eng E;                                                                      \
     E.init(s, A.tw);
