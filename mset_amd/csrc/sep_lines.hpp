@@ -43,7 +43,9 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int N> struct SepLines {
+// BUF plane buffers: with two, a turn writes the one that the turn before last was read from, and needs one barrier
+// (one-position kernel, 64 x 64, 16 planes: 145 -> 141 us; batches at 48, where it costs a workgroup per CU: 206 -> 259).
+template <int N, int BUF> struct SepLines {
     using P = SepPlan<N>;
     static constexpr int R1 = P::R1, R2 = P::R2, T = P::T;
     static constexpr int NT = N * T;
@@ -54,11 +56,12 @@ template <int N> struct SepLines {
     // the plane and the exchange slots are apart where both fit beside a second workgroup, else they share
     static constexpr bool APART = N <= 64;
     static constexpr int EX_ELEMS = N * LS, PL_ELEMS = N * PITCH;
-    static constexpr int LDS_ELEMS = APART ? EX_ELEMS + PL_ELEMS : (EX_ELEMS > PL_ELEMS ? EX_ELEMS : PL_ELEMS);
+    static constexpr int LDS_ELEMS = APART ? EX_ELEMS + BUF * PL_ELEMS : (EX_ELEMS > PL_ELEMS ? EX_ELEMS : PL_ELEMS);
+    static_assert(BUF == 1 || APART, "a second buffer beside the exchange slots");
     static_assert(N == R1 * R2 && R2 <= T && 64 % T == 0, "a line's lanes are in one wave");
 
     float2* lds;
-    int line, j;
+    int line, j, pl;     // pl: the plane buffer of the next turn
     float2 w[R1 - 1];    // W_N^(j k1), k1 = 1 .. R1 - 1
     float2 v[EM];
 
@@ -66,12 +69,16 @@ template <int N> struct SepLines {
         lds = s;
         line = threadIdx.x / T;
         j = threadIdx.x % T;
+        pl = APART ? EX_ELEMS : 0;
 #pragma unroll
         for (int k = 1; k < R1; ++k) w[k - 1] = tw[jd() * k % N];
     }
     // Addresses are affine in (line, j); left visible, the compiler hoists them all out of the plane loops and keeps
     // a hundred registers live (see RegEngine::opaque)
-    __device__ __forceinline__ void opaque() { asm volatile("" : "+v"(line), "+v"(j)); }
+    __device__ __forceinline__ void opaque() {
+        asm volatile("" : "+v"(line), "+v"(j));
+        __builtin_assume(line >= 0 && line < N && j >= 0 && j < T);   // 24-bit multiplies and shifts
+    }
     // Where a layout has fewer places than lanes (j >= R2 in D, j + c T >= R1 in X), the lanes beyond the last place
     // duplicate it: same point, same values, same addresses written, so no access needs a mask or a branch.  Sums over
     // the points leave them out (own_x, own_d).
@@ -82,7 +89,7 @@ template <int N> struct SepLines {
 
     __device__ __forceinline__ void fwd() {
         opaque();
-        float2* ex = lds + __mul24(line, LS);               // this line's exchange slots
+        float2* ex = lds + line * LS;                       // this line's exchange slots
         DFT<R1, false>::run(v);
 #pragma unroll
         for (int k = 1; k < R1; ++k) v[k] = cmul(v[k], w[k - 1]);
@@ -91,7 +98,7 @@ template <int N> struct SepLines {
         wave_lds_fence();
 #pragma unroll
         for (int c = 0; c < CX; ++c) {
-            const float2* q = ex + __mul24(jx(c), EXP);
+            const float2* q = ex + jx(c) * EXP;
 #pragma unroll
             for (int i = 0; i < R2; ++i) v[c * R2 + i] = q[i];
         }
@@ -101,12 +108,12 @@ template <int N> struct SepLines {
     }
     __device__ __forceinline__ void inv() {
         opaque();
-        float2* ex = lds + __mul24(line, LS);
+        float2* ex = lds + line * LS;
 #pragma unroll
         for (int c = 0; c < CX; ++c) DFT<R2, true>::run(v + c * R2);
 #pragma unroll
         for (int c = 0; c < CX; ++c) {
-            float2* q = ex + __mul24(jx(c), EXP);
+            float2* q = ex + jx(c) * EXP;
 #pragma unroll
             for (int i = 0; i < R2; ++i) q[i] = v[c * R2 + i];
         }
@@ -136,15 +143,16 @@ template <int N> struct SepLines {
     // turns the plane over: layout D or X of lines along one axis -> layout D or X of lines along the other.
     // col: the lines written are columns x (points y).
     template <bool FROM_X, bool TO_X> __device__ __forceinline__ void turn(bool col) {
-        __syncthreads();                                     // the plane slots were read (and, shared, exchanged in)
+        if constexpr (BUF == 1) __syncthreads();             // the plane slots were read (and, shared, exchanged in)
         opaque();
-        float2* pl = lds + (APART ? EX_ELEMS : 0);
+        float2* pl = lds + this->pl;
+        if constexpr (BUF == 2) this->pl = 2 * EX_ELEMS + PL_ELEMS - this->pl;
         const int wl = col ? 1 : PITCH, wp = col ? PITCH : 1;
-        auto put = [&](int i, int p, int q) { (pl + __mul24(line, wl) + __mul24(p, wp))[q * wp] = v[i]; };
+        auto put = [&](int i, int p, int q) { (pl + line * wl + p * wp)[q * wp] = v[i]; };
         if constexpr (FROM_X) each_x(put);
         else each_d(put);
         __syncthreads();
-        auto get = [&](int i, int p, int q) { v[i] = (pl + __mul24(line, wp) + __mul24(p, wl))[q * wl]; };
+        auto get = [&](int i, int p, int q) { v[i] = (pl + line * wp + p * wl)[q * wl]; };
         if constexpr (TO_X) each_x(get);
         else each_d(get);
         if constexpr (!APART) __syncthreads();               // before exchanges write the shared slots
@@ -154,10 +162,10 @@ template <int N> struct SepLines {
 // One probe position: K_BATCH (gradient terms into slabs), K_FWD (loss) or K_PLAIN (sequential semantics; gradient
 // planes to slab 0, probe and position updated).  Reference pairing, stored waves, multislice operator; passes
 // X_0 .. X_(2L+3) and scratch planes as in process_sep, all arrays in the layouts of process_position.
-template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(const PosArgs& A, int k, int slot, int slab,
-                                                                               bool first, SepLines<N>& E, float2* phx, float2* phy,
+template <int N, int KIND, int BUF> __device__ __forceinline__ void position_sep_lines(const PosArgs& A, int k, int slot, int slab,
+                                                                               bool first, SepLines<N, BUF>& E, float2* phx, float2* phy,
                                                                                const float2* px, const float2* py, double* red) {
-    using Eng = SepLines<N>;
+    using Eng = SepLines<N, BUF>;
     constexpr int N2 = N * N, R1 = Eng::R1, R2 = Eng::R2, EM = Eng::EM, NT = Eng::NT;
     constexpr bool GRAD = KIND != K_FWD;
     const int t = threadIdx.x, L = A.L;
@@ -181,7 +189,7 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
     // index of point p + q of the line in a row-major [y][x] array (rm) and in a transposed [x][y] one (tm): the lane's
     // part and the register's (a constant for each orientation)
     auto rm = [&](bool col, int p, int q) {
-        return Idx{(unsigned)(__mul24(E.line, col ? 1 : N) + __mul24(p, col ? N : 1)), (unsigned)(q * (col ? N : 1))};
+        return Idx{(unsigned)(E.line * (col ? 1 : N) + p * (col ? N : 1)), (unsigned)(q * (col ? N : 1))};
     };
     auto tm = [&](bool col, int p, int q) { return rm(!col, p, q); };
     auto rm_d = [&](bool col, int r) { return rm(col, E.jd(), r * R2); };
@@ -251,10 +259,15 @@ template <int N, int KIND> __device__ __forceinline__ void position_sep_lines(co
         E.inv();
         E.template turn<false, false>(col);
     };
-    // a pass of each orientation: strides and offsets are constants
-    for (int a = 1; a < L; a += 2) {
-        plane_fwd(true, a);
-        if (a + 1 < L) plane_fwd(false, a + 1);
+    // a pass of each orientation per round, strides and offsets constants; without a gradient from 96 on one body
+    // (fewer spilled registers; 128, 12 planes of 700 positions: 545 us against 560)
+    if constexpr (KIND != K_FWD || N < 96) {
+        for (int a = 1; a < L; a += 2) {
+            plane_fwd(true, a);
+            if (a + 1 < L) plane_fwd(false, a + 1);
+        }
+    } else {
+        for (int a = 1; a < L; ++a) plane_fwd(a & 1, a);
     }
     // ---- X_(L+1): finish plane L-1's step, keep psi_L, forward along this axis
     float m[EM];
@@ -393,12 +406,12 @@ __device__ __forceinline__ int slab_of(int p, int nslab) { return __builtin_amdg
 
 // registers for two workgroups per CU at 64, where LDS holds two, and for one of 1024 threads at 128
 template <int N> struct SepCfg {
-    static constexpr int NT = SepLines<N>::NT;
+    static constexpr int NT = SepLines<N, 1>::NT;
     static constexpr int MINB = N == 64 || N == 128 ? 4 : N == 96 ? 3 : 1;
 };
 
-#define MSET_SEP_LDS(N)                                                         \
-    using Eng = SepLines<N>;                                                        \
+#define MSET_SEP_LDS(N, BUF)                                                    \
+    using Eng = SepLines<N, BUF>;                                               \
     constexpr int NT = Eng::NT;                                                 \
     __shared__ float2 s[Eng::LDS_ELEMS];                                        \
     __shared__ float2 phx[N], phy[N], px[N], py[N];                             \
@@ -409,7 +422,7 @@ template <int N> struct SepCfg {
     E.init(s, A.tw);
 
 template <int N> __global__ __launch_bounds__((SepCfg<N>::NT), (SepCfg<N>::MINB)) void k_sep_batch(PosArgs A) {
-    MSET_SEP_LDS(N)
+    MSET_SEP_LDS(N, (N <= 32 ? 2 : 1))
     for (int p = blockIdx.x; p < A.count; p += gridDim.x) {
         const int k = A.order ? A.order[A.first + p] : A.first + p;
         position_sep_lines<N, K_BATCH>(A, k, blockIdx.x, slab_of(p, A.nslab), p < A.nslab, E, phx, phy, px, py, red);
@@ -417,13 +430,13 @@ template <int N> __global__ __launch_bounds__((SepCfg<N>::NT), (SepCfg<N>::MINB)
 }
 
 template <int N> __global__ __launch_bounds__((SepCfg<N>::NT), (SepCfg<N>::MINB)) void k_sep_plain(PosArgs A, int k) {
-    MSET_SEP_LDS(N)
+    MSET_SEP_LDS(N, (N <= 64 ? 2 : 1))
     position_sep_lines<N, K_PLAIN>(A, k, 0, 0, true, E, phx, phy, px, py, red);
 }
 
 // MT: the work items are positions of several tilts (as k_fwd)
 template <int N, bool MT> __global__ __launch_bounds__((SepCfg<N>::NT), (SepCfg<N>::MINB)) void k_sep_fwd(PosArgs A) {
-    MSET_SEP_LDS(N)
+    MSET_SEP_LDS(N, (N <= 32 ? 2 : 1))
     for (int p = blockIdx.x; p < A.count; p += gridDim.x) {
         if constexpr (MT) {
             const int item = A.order[p];
