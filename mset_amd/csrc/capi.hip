@@ -288,9 +288,9 @@ bool sep_batch(const mset_ctx* c) {
 
 // The on-chip separable routine (sep_lines.hpp): forward-only launches below 256, gradients and the one-position
 // kernel with the reference pairing and stored waves below 128.  12 planes, the LDS engine against it, gradient
-// and forward-only: 256 positions 43 -> 35 and 24 -> 18 us at 16, 67 -> 63 and 35 -> 30 at 24, 73 -> 63 and 37 -> 33 at
-// 32, 131 -> 94 and 65 -> 41 at 48, 167 -> 132 and 74 -> 49 at 64, 440 -> 330 and 181 -> 121 at 96; 1400 positions
-// 54 -> 43, 137 -> 115, 167 -> 156, 652 -> 413, 787 -> 673 us (700 at 96: 1286 -> 995).  At 128, 16 planes, 1024 positions:
+// and forward-only: 256 positions 43 -> 33 and 24 -> 18 us at 16, 67 -> 51 and 35 -> 27 at 24, 73 -> 60 and 37 -> 30 at
+// 32, 131 -> 93 and 65 -> 43 at 48, 167 -> 131 and 74 -> 50 at 64, 440 -> 329 and 181 -> 122 at 96; 700 at 96 1286 -> 985;
+// 1400 positions 54 -> 43, 137 -> 115, 167 -> 156, 652 -> 413, 787 -> 673 us at 16 .. 64.  At 128, 16 planes, 1024 positions:
 // forward-only 1188 -> 958 us against the register engine, the gradient 2838 -> 2846 (its operands leave too few
 // registers), so that stays there.
 bool sep_fwd_lines(const mset_ctx* c) {
@@ -455,7 +455,7 @@ int read_errors(mset_ctx* c, int first, int count, double* out) {
 
 // The sequential path as line passes over the whole device (line_passes.hip): a separable propagator, the
 // reference pairing, from 96 x 96 up.  Both ways cost about the same per plane at any depth; per position, one
-// workgroup of the on-chip separable routine against line passes: 71 and 70 us at 64 x 64 (6 planes; 149 and 159
+// workgroup of the on-chip separable routine against line passes: 67 and 70 us at 64 x 64 (6 planes; 139 and 159
 // with 16), 166 and 91 us at 96 x 96 (6), 267 and 94 us at 128 x 128 (6).
 bool plain_lines(const mset_ctx* c) {
     return position_lines_supported(c->n) && c->prop_sep && !sset(c) && c->p.grad_mode == GRAD_REF &&
@@ -466,7 +466,7 @@ bool plain_lines(const mset_ctx* c) {
 int issue_plain(mset_ctx* c) {
     CHK(c->ws->save.ensure((size_t)(c->L + 2) * plane(c), "save waves"));
     if (plain_lines(c)) {
-        CHK(c->ws->lines.ensure(position_lines_work(c->n), "line passes"));
+        CHK(c->ws->lines.ensure(position_lines_work(c->n, c->L), "line passes"));
         const PosArgs P = base_args(c);
         for (int k = 0; k < c->npos; ++k) {
             Timed t(c, "position_plain");

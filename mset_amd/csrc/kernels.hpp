@@ -87,6 +87,7 @@ struct LineArgs {
     const float2* p1d;           // propagator factors px[N], py[N]
     float2* phi;                 // sub-pixel shift factors along x [N], along y [N]
     float* V;                    // volume [z][y][x]
+    float2* trans;               // the plane's transmission, lines of its forward pass contiguous
     float2* wave;                // psi of the pass's plane, lines contiguous (written forward, read back)
     const float2* psi0;          // incident wave [y][x]
     float2* probe;               // [y][x]
@@ -104,9 +105,9 @@ bool plane_size_supported(int n);
 int position_threads(int n);
 hipError_t launch_plain(int n, const PosArgs& A, int k, hipStream_t st);
 // sequential path as line passes over the device (separable propagator, reference pairing): position k of P
-// with V, the probe and the position updated; work: position_lines_work(n) elements
+// with V, the probe and the position updated; work: position_lines_work(n, L) elements
 bool position_lines_supported(int n);
-size_t position_lines_work(int n);
+size_t position_lines_work(int n, int L);
 hipError_t launch_position_lines(int n, const PosArgs& P, int k, float2* work, hipStream_t st);
 // shape: 0 default, 1 alternative (MSET_ENGINE_ALT_SHAPE, stored waves), 2 the large workgroup for launches of
 // at most one position per CU (at 48 with stored waves; the separable 256 routine, stored or checkpointed)

@@ -29,12 +29,14 @@
 //   ADJ    both     half-step back, gradient, V += s1 G, x conj(t_a), half-step back     a = L-1 .. 0
 //   BACK   rows     F -> fftn(bw), x conj(Phi), F^-1
 //   STEP   columns  F^-1 -> probe -= s2 w, position += s3 d
-// V is read where a plane is used and updated in its adjoint pass, after which the position does not read
-// it again, so there are no transmission planes, gradient planes or update launches.  Waves, loss and
+// V is read in a plane's forward pass, which keeps the transmission for the adjoint one, and updated in its adjoint
+// pass, so there are no gradient planes, transmission or update launches.  (Forming the transmission again in the
+// adjoint pass: 7.56 instead of 7.28 ms for 36 positions at 128 x 128 x 16 planes; with views instead of pointers and
+// no branch around the slices 6.63 ms.)  Waves, loss and
 // position sums, rounding order of the transmission and the update as in process_position.
 //
-// Measured per position, before as one workgroup and now: 576 -> 205 us at 128 x 128 x 16 planes (38 launches),
-// 4.5 -> 0.45 ms at 256 x 256 x 32 (70); a pass with four transforms takes 5 to 6 us at 128, about 2 of them the
+// Measured per position, before as one workgroup and now: 576 -> 184 us at 128 x 128 x 16 planes (38 launches),
+// 4.5 -> 0.45 ms at 256 x 256 x 32 (70); a pass with four transforms takes about 5 us at 128, about 2 of them the
 // launch and the loads.
 #include <hip/hip_runtime.h>
 
@@ -75,58 +77,72 @@ template <int N, int KIND, bool COL> __global__ __launch_bounds__(N) void k_line
     F_ F;
     F.init(s, A.tw);
     const int line = blockIdx.x * TL + F.line, j = F.j;
-    // index of point r of the thread in arrays with contiguous lines, and in arrays of the other orientation
-    auto own = [&](int r) { return line * N + j + r * T; };
-    auto oth = [&](int r) { return (j + r * T) * N + line; };
+    // index of point r of the thread in arrays with contiguous lines, and in arrays of the other orientation: the
+    // thread's part and a constant, through buffer views (with pointers a pass formed 26 addresses by 64-bit multiplies)
+    auto own = [&](int r) { return Idx{(unsigned)(line * N + j), (unsigned)(r * T)}; };
+    auto oth = [&](int r) { return Idx{(unsigned)(j * N + line), (unsigned)(r * T * N)}; };
+    auto along = [&](int r) { return Idx{(unsigned)j, (unsigned)(r * T)}; };
+    const BufC in(A.in, N2), out(A.out, N2), wave(A.wave, N2), trans(A.trans, N2);
     const float inv_n = 1.0f / (float)N, inv_n2 = 1.0f / (float)N2;
 
     // ---- operands, all requested before the first transform
     float2 v[E];
 #pragma unroll
-    for (int r = 0; r < E; ++r) v[r] = A.in[own(r)];
+    for (int r = 0; r < E; ++r) v[r] = in[own(r)];
     // propagator factors along the pass
     float2 pf[E];
     if constexpr (KIND == FIRST || KIND == FWD || KIND == LAST || KIND == EXIT || KIND == ADJ) {
+        const BufC f(A.p1d + (COL ? N : 0), N);
 #pragma unroll
-        for (int r = 0; r < E; ++r) pf[r] = A.p1d[(COL ? N : 0) + j + r * T];
+        for (int r = 0; r < E; ++r) pf[r] = f[along(r)];
     }
-    // the plane's slices: the first four kept for the update, the sum in slice order
+    // the plane's slices: the first four kept for the update, the sum in slice order.  A slice beyond the bin has an
+    // empty view (reads 0, drops writes): with a branch around its loads the compiler moved the first addition up to
+    // the load, and the pass waited for memory before its first transform.
     constexpr int KEEP = 4;
     float z[KEEP][E], sum[E];
-    const int z0 = A.a * A.bin, nzp = min(A.bin, A.nz - z0);
+    // (without an object step the adjoint pass has no slices)
+    const int z0 = A.a * A.bin, nzp = KIND == ADJ && A.s1 == 0.f ? 0 : min(A.bin, A.nz - z0);
     float* Vp = A.V + (size_t)z0 * N2;
+    auto slice = [&](int i) { return BufF(Vp + (size_t)i * N2, i < nzp ? (unsigned)N2 : 0u); };
+    auto vox = [&](int r) { return COL ? oth(r) : own(r); };
     if constexpr (KIND == FIRST || KIND == FWD || KIND == ADJ) {
 #pragma unroll
         for (int r = 0; r < E; ++r) sum[r] = 0.f;
 #pragma unroll
-        for (int i = 0; i < KEEP; ++i)
-            if (i < nzp) {
+        for (int i = 0; i < KEEP; ++i) {
+            const BufF V = slice(i);
 #pragma unroll
-                for (int r = 0; r < E; ++r) z[i][r] = Vp[(size_t)i * N2 + (COL ? oth(r) : own(r))];
-            }
+            for (int r = 0; r < E; ++r) z[i][r] = V[vox(r)];
+        }
     }
-    float2 wv[E];
+    float2 wv[E], t[E];
     if constexpr (KIND == ADJ) {
 #pragma unroll
-        for (int r = 0; r < E; ++r) wv[r] = A.wave[own(r)];
+        for (int r = 0; r < E; ++r) wv[r] = wave[own(r)];
+#pragma unroll
+        for (int r = 0; r < E; ++r) t[r] = trans[oth(r)];
     }
     float m[E];
     if constexpr (KIND == EXIT) {
+        const BufF M(A.sqrtM, N2);
 #pragma unroll
-        for (int r = 0; r < E; ++r) m[r] = A.sqrtM[COL ? own(r) : oth(r)];
+        for (int r = 0; r < E; ++r) m[r] = M[COL ? own(r) : oth(r)];
     }
     float2 pr[E];
+    const BufC probe(A.probe, N2);
     if constexpr (KIND == STEP) {
 #pragma unroll
-        for (int r = 0; r < E; ++r) pr[r] = A.probe[COL ? oth(r) : own(r)];
+        for (int r = 0; r < E; ++r) pr[r] = probe[vox(r)];
     }
     // sub-pixel shift factors: phi[0 .. N) along x, phi[N .. 2N) along y
     float2 ph[E];
     if constexpr (KIND == SHIFT || KIND == BACK) {
         const float2 l = A.phi[(COL ? 0 : N) + line];
+        const BufC f(A.phi + (COL ? N : 0), N);
 #pragma unroll
         for (int r = 0; r < E; ++r) {
-            const float2 q = A.phi[(COL ? N : 0) + j + r * T];
+            const float2 q = f[along(r)];
             ph[r] = COL ? cmul(q, l) : cmul(l, q);               // phy * phx
         }
     }
@@ -143,24 +159,25 @@ template <int N, int KIND, bool COL> __global__ __launch_bounds__(N) void k_line
         }
     }
     // transmission of the plane (STEP02_FORWARD_4D.m:18-19 rounding order), formed where it is applied so
-    // that the wait for the slices falls behind the first transforms
-    float2 t[E];
+    // that the wait for the slices falls behind the first transforms, and kept for the adjoint pass (which runs along
+    // the other axis)
     auto transmission = [&]() {
 #pragma unroll
-        for (int i = 0; i < KEEP; ++i)
-            if (i < nzp) {
+        for (int i = 0; i < KEEP; ++i) {
 #pragma unroll
-                for (int r = 0; r < E; ++r) sum[r] += z[i][r];
-            }
+            for (int r = 0; r < E; ++r) sum[r] += z[i][r];
+        }
         for (int i = KEEP; i < nzp; ++i) {
+            const BufF V = slice(i);
 #pragma unroll
-            for (int r = 0; r < E; ++r) sum[r] += Vp[(size_t)i * N2 + (COL ? oth(r) : own(r))];
+            for (int r = 0; r < E; ++r) sum[r] += V[vox(r)];
         }
 #pragma unroll
         for (int r = 0; r < E; ++r) {
             float sn, cs;
             sincosf(A.sigma * (sum[r] * A.dx), &sn, &cs);
             t[r] = make_float2(cs, sn);
+            trans.put(own(r), t[r]);
         }
     };
 
@@ -186,7 +203,7 @@ template <int N, int KIND, bool COL> __global__ __launch_bounds__(N) void k_line
 #pragma unroll
         for (int r = 0; r < E; ++r) {
             if constexpr (KIND == FIRST) v[r] = cscale(v[r], inv_n2);
-            A.wave[own(r)] = v[r];
+            wave.put(own(r), v[r]);
         }
         if constexpr (KIND != LAST) {
             transmission();
@@ -225,7 +242,6 @@ template <int N, int KIND, bool COL> __global__ __launch_bounds__(N) void k_line
             F.template dft<true>(v);
         }
         // gradient (STEP03_BACK.m:12-24), the object step of every slice of the bin (:84), x conj(t)
-        transmission();
         float g[E];
 #pragma unroll
         for (int r = 0; r < E; ++r) {
@@ -233,17 +249,16 @@ template <int N, int KIND, bool COL> __global__ __launch_bounds__(N) void k_line
             g[r] = -cmul(tc, cmulc(v[r], wv[r])).y;                  // Re(1i * conj(t) * conj(psi) * b)
             v[r] = cmul(v[r], tc);
         }
-        if (A.s1 != 0.f) {
 #pragma unroll
-            for (int i = 0; i < KEEP; ++i)
-                if (i < nzp) {
+        for (int i = 0; i < KEEP; ++i) {
+            const BufF V = slice(i);
 #pragma unroll
-                    for (int r = 0; r < E; ++r) Vp[(size_t)i * N2 + (COL ? oth(r) : own(r))] = z[i][r] + A.s1 * g[r];
-                }
-            for (int i = KEEP; i < nzp; ++i) {
+            for (int r = 0; r < E; ++r) V.put(vox(r), z[i][r] + A.s1 * g[r]);
+        }
+        for (int i = KEEP; i < nzp; ++i) {
+            const BufF V = slice(i);
 #pragma unroll
-                for (int r = 0; r < E; ++r) Vp[(size_t)i * N2 + (COL ? oth(r) : own(r))] += A.s1 * g[r];
-            }
+            for (int r = 0; r < E; ++r) V.put(vox(r), V[vox(r)] + A.s1 * g[r]);
         }
         if constexpr (COL) {
             if (A.a == 0 && A.want_pos) {
@@ -291,18 +306,18 @@ template <int N, int KIND, bool COL> __global__ __launch_bounds__(N) void k_line
         if (A.s2 == 0.f) return;
         F.template dft<true>(v);
 #pragma unroll
-        for (int r = 0; r < E; ++r) A.probe[COL ? oth(r) : own(r)] = csub(pr[r], cscale(cscale(v[r], inv_n2), A.s2));
+        for (int r = 0; r < E; ++r) probe.put(vox(r), csub(pr[r], cscale(cscale(v[r], inv_n2), A.s2)));
         return;
     }
     // transposed: the next pass runs along the other axis
 #pragma unroll
-    for (int r = 0; r < E; ++r) A.out[oth(r)] = v[r];
+    for (int r = 0; r < E; ++r) out.put(oth(r), v[r]);
 }
 
 template <int N> hipError_t position_lines(const PosArgs& P, int k, float2* work, hipStream_t st) {
     constexpr int N2 = N * N;
     const int L = P.L;
-    float2 *a = work, *b = work + N2;
+    float2 *a = work, *b = work + N2, *trans = work + position_lines_work(N, 0);
     LineArgs A{};
     A.tw = P.tw;
     A.p1d = P.p1d;
@@ -345,11 +360,13 @@ template <int N> hipError_t position_lines(const PosArgs& P, int k, float2* work
     MSET_LINE(SHIFT, true);
     next();
     A.wave = P.save;
+    A.trans = trans;
     MSET_LINE(FIRST, false);
     for (int i = 1; i < L; ++i) {
         next();
         A.a = i;
         A.wave = P.save + (size_t)i * N2;
+        A.trans = trans + (size_t)i * N2;
         MSET_LINE2(FWD, i % 2 == 1);
     }
     next();
@@ -361,6 +378,7 @@ template <int N> hipError_t position_lines(const PosArgs& P, int k, float2* work
         next();
         A.a = i;
         A.head = i == L - 1;
+        A.trans = trans + (size_t)i * N2;
         A.wave = P.save + (size_t)(i + 1) * N2;                 // reference pairing: the wave after plane i
         MSET_LINE2(ADJ, i % 2 == 0);
     }
@@ -381,8 +399,8 @@ template <int N> hipError_t position_lines(const PosArgs& P, int k, float2* work
 
 bool position_lines_supported(int n) { return n == 96 || n == 128 || n == 256; }
 
-// two plane buffers, the shift factors and three sums per workgroup
-size_t position_lines_work(int n) { return 2 * (size_t)n * n + 2 * (size_t)n + 3 * (size_t)(n / TL); }
+// two plane buffers, the shift factors, three sums per workgroup, the transmission planes
+size_t position_lines_work(int n, int L) { return (2 + (size_t)L) * n * n + 2 * (size_t)n + 3 * (size_t)(n / TL); }
 
 hipError_t launch_position_lines(int n, const PosArgs& P, int k, float2* work, hipStream_t st) {
     switch (n) {
