@@ -156,7 +156,7 @@ int mset_set_slot_limit(mset_ctx* ctx, int slots);
  * waves run the separable routine, which applies the two 1D half-steps of neighbouring planes in one pass
  * over the plane (half the passes).  GENERAL: always the 2D routine.  ALT_SHAPE: the batched kernel with
  * stored waves runs the alternative workgroup shape of its plane size: fewer threads per position of the LDS
- * engine at 24, 32, 64 and 96 (more at 16 and 48), at 128 the register engine with a half-size transpose
+ * engine at 24, 32, 64 and 96 (more at 48, as many at 16), at 128 the register engine with a half-size transpose
  * buffer and a 128-register budget (two workgroups per CU instead of one), at 256 16-line tiles with 256
  * threads (three workgroups per CU instead of two).  The flags combine. */
 #define MSET_ENGINE_AUTO 0

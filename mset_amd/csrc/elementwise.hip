@@ -60,8 +60,8 @@ __global__ __launch_bounds__(256) void k_volume(float* V, const float* __restric
 }
 
 // Transmission phases for the separable-propagator kernels, which form t = exp(i pi r) where they apply it
-// (half the bytes of a complex plane).  r is the f32 phase of k_trans, divided by pi and reduced to [-1, 1]
-// in double: t differs from k_trans's sincosf by about 1e-7.  Plane a goes to Tf in the
+// (half the bytes of a complex plane).  r is the f32 phase of k_volume, divided by pi and reduced to [-1, 1]
+// in double: t differs from k_volume's sincosf by about 1e-7.  Plane a goes to Tf in the
 // layout of the pass that applies it in the forward sweep (rows, [x][y], for even a; columns, [y][x], for
 // odd a) and, if Tb is given, to Tb in the layout of its adjoint pass (the other one).
 __global__ void k_trans_sep(const float* __restrict__ V, float* __restrict__ Tf, float* __restrict__ Tb, int n, int nz,

@@ -1,6 +1,6 @@
 // multislice.hpp -- fused multislice forward / adjoint kernels (CDNA4, gfx950): the position routines
-// and the kernel templates.  The launchers instantiate them in three translation units (multislice.hip:
-// sequential, forward-only and plane-FFT kernels; batch_store.hip: the batched gradient with stored waves;
+// and the kernel templates.  The launchers instantiate them in four translation units (multislice.hip:
+// sequential and plane-FFT kernels; forward.hip: forward-only; batch_store.hip: the batched gradient with stored waves;
 // batch_variants.hip: with recomputed or checkpointed waves), so that the build compiles them in parallel.
 //
 // One workgroup owns one probe position at a time and keeps the N x N wave in LDS for the whole
