@@ -471,18 +471,24 @@ __device__ __forceinline__ void process_position(const PosArgs& A, int k, int sl
             // back_wave_f = ifftn(B); MATLAB gradient() of conj(psi0), one-sided at the edges
             E.inv(NoOp(), [&](const Pt&, float2 v) { return cscale(v, inv_n2); });
             have_bw = true;
-            const float2* p0 = save;
-            E.each_C([&](const Pt& p, float2& bw) {
-                const int y = p.y, x = p.x;
-                // clamped neighbours: the edge rows / columns become the one-sided differences
-                const int xp = min(x + 1, N - 1), xm = max(x - 1, 0);
-                const int yp = min(y + 1, N - 1), ym = max(y - 1, 0);
-                const float2 gx = cscale(csub(p0[y * N + xp], p0[y * N + xm]), xp - xm == 2 ? 0.5f : 1.0f);
-                const float2 gy = cscale(csub(p0[yp * N + x], p0[ym * N + x]), yp - ym == 2 ? 0.5f : 1.0f);
-                // Re(conj(g) * bw)
-                dr += (double)(gx.x * bw.x + gx.y * bw.y);
-                dc += (double)(gy.x * bw.x + gy.y * bw.y);
-            });
+            // (clamped neighbours: the edge rows / columns become the one-sided differences), 8 points' neighbours in
+            // flight: one by one they cost two memory latencies a point (1024 positions at 128 x 128 x 16: 3.39 -> 3.35 ms)
+            struct Nb {
+                float2 xp, xm, yp, ym;
+            };
+            E.each_C(staged<8>(
+                [&](const Pt& p) {
+                    const int y = p.y, x = p.x;
+                    auto at = [&](int yy, int xx) { return sv0[Idx{(unsigned)(yy * N + xx), 0}]; };
+                    return Nb{at(y, min(x + 1, N - 1)), at(y, max(x - 1, 0)), at(min(y + 1, N - 1), x), at(max(y - 1, 0), x)};
+                },
+                [&](const Pt& p, float2& bw, const Nb& o) {
+                    const float2 gx = cscale(csub(o.xp, o.xm), p.x > 0 && p.x < N - 1 ? 0.5f : 1.0f);
+                    const float2 gy = cscale(csub(o.yp, o.ym), p.y > 0 && p.y < N - 1 ? 0.5f : 1.0f);
+                    // Re(conj(g) * bw)
+                    dr += (double)(gx.x * bw.x + gx.y * bw.y);
+                    dc += (double)(gy.x * bw.x + gy.y * bw.y);
+                }));
             dr = block_sum<NT>(dr, red);
             dc = block_sum<NT>(dc, red);
         }
