@@ -72,7 +72,7 @@ template <> struct Cfg<32, 1> { static constexpr int NT = 64, MINB = 1; using En
 template <> struct Cfg<48, 1> { static constexpr int NT = 384, MINB = 1; using Eng = LdsEngine<48, 384>; };
 template <> struct Cfg<64, 1> { static constexpr int NT = 256, MINB = 3; using Eng = LdsEngine<64, 256>; };
 template <> struct Cfg<96, 1> { static constexpr int NT = 576, MINB = 1; using Eng = LdsEngine<96, 576>; };
-template <> struct Cfg<128, 1> { static constexpr int NT = 512, MINB = 4; using Eng = RegEngine<128>; };
+template <> struct Cfg<128, 1> { static constexpr int NT = 512, MINB = 4; using Eng = RegEngine<128, true>; };
 template <> struct Cfg<256, 1> { static constexpr int NT = 256, MINB = 3; using Eng = TiledEngine<256, 256>; };
 template <int N> struct Cfg<N, 2> : Cfg<N> {};
 template <> struct Cfg<48, 2> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<48, 768>; };
