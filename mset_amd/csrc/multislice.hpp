@@ -52,7 +52,7 @@ namespace mset {
 // the exact pairing, recomputed and checkpointed waves, other propagators, the single-slice operator.
 // SH = 1: the alternative shape of the batched kernel, a candidate for the autotuner (MSET_ENGINE_ALT_SHAPE):
 // smaller workgroups below 128 (at 48 a larger one); at 128 the register engine with a half-size transpose buffer
-// and a 128-register budget (two workgroups per CU instead of one; it spills about 400 registers); tiles of 16 lines
+// and a 128-register budget (two workgroups per CU instead of one; it spills about 340 registers); tiles of 16 lines
 // with 256 threads (three workgroups per CU instead of two) at 256.
 // SH = 2: launches of at most one position per CU and the one-position kernel: at 48 a workgroup of 768, at 256
 // 64-line tiles, one workgroup of 16 waves per CU with twice the default workgroup's loads in flight; the
