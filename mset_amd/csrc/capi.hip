@@ -52,12 +52,16 @@ int fail(int code, const std::string& msg) {
 template <typename T> struct DevBuf {
     T* p = nullptr;
     size_t n = 0;
+    unsigned freed = 0;              // allocations given back so far (a captured pass may hold one of them)
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) {
+            (void)hipFree(p);
+            ++freed;
+        }
         p = nullptr;
         n = 0;
     }
@@ -95,6 +99,11 @@ struct Workspace {
     size_t slot_bytes = 0;                   // its per-slot scratch (waves + gradient slab)
     RotWork rot;
     TvWork tv;
+    // allocations given back by the buffers an update pass uses: a pass captured at another count holds freed memory
+    unsigned long long freed() const {
+        return 0ull + save.freed + trans.freed + probeF.freed + pslab.freed + PG.freed + planes.freed + lines.freed +
+               gslab.freed + G.freed + rot.freed;
+    }
     ~Workspace() {
         rot_release(rot);
         tv_release(tv);
@@ -738,6 +747,7 @@ struct mset_recon {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int graph_key[3] = {-1, -1, -1};
+    unsigned long long graph_freed = 0;   // ws->freed() when the pass was captured
     // the error pass over every tilt in one launch: per-tilt table, work items, per-position errors
     DevBuf<TiltArgs> tilt_tab;
     DevBuf<int> items;
@@ -1233,7 +1243,9 @@ int mset_recon_iterate(mset_recon* r, int path, int batch, int use_graph, int po
     if (path == MSET_PATH_BATCHED && batch <= 0) return fail(MSET_EINVAL, "batch must be positive");
     if (path == MSET_PATH_PLAIN) batch = 1;
     if (use_graph && !r->profiling && (path != MSET_PATH_PLAIN || plain_launches(r) <= PLAIN_GRAPH_LAUNCHES)) {
-        const bool same = r->exec && r->graph_key[0] == path && r->graph_key[1] == batch && r->graph_key[2] == positivity;
+        // an eager pass, or an error pass, may have reallocated a buffer that the captured pass holds
+        const bool same = r->exec && r->graph_key[0] == path && r->graph_key[1] == batch && r->graph_key[2] == positivity &&
+                          r->graph_freed == r->ws->freed();
         if (!same) {
             drop_graph(r);
             // eager pass first: every allocation and twiddle upload happens outside the capture
@@ -1253,6 +1265,7 @@ int mset_recon_iterate(mset_recon* r, int path, int batch, int use_graph, int po
             r->graph_key[0] = path;
             r->graph_key[1] = batch;
             r->graph_key[2] = positivity;
+            r->graph_freed = r->ws->freed();
             // the eager pass above was this call's iteration
         } else {
             HIPCHK(hipGraphLaunch(r->exec, r->stream));
@@ -1297,11 +1310,7 @@ int mset_recon_error_pass(mset_recon* r, double* errs) {
     int grid = std::max(1, device_slots(c0, 0));
     if (r->ws->slot_limit > 0) grid = std::min(grid, r->ws->slot_limit);
     grid = (int)std::min<size_t>((size_t)grid, tot);
-    if (plane_in_global(r->n)) {
-        const size_t need = (size_t)grid * 2 * plane(c0);
-        if (r->ws->planes.n < need) drop_graph(r);       // a captured update pass holds the current buffer
-        CHK(r->ws->planes.ensure(need, "plane buffers"));
-    }
+    if (plane_in_global(r->n)) CHK(r->ws->planes.ensure((size_t)grid * 2 * plane(c0), "plane buffers"));
     std::vector<TiltArgs> tab(T);
     std::vector<int> items(tot);
     const bool sep = sep_fwd(c0);

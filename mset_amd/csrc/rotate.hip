@@ -635,7 +635,10 @@ int run_planar(RotWork& W, const std::vector<PlanarShear>& shears, int third, co
     const int pb = third == 0 ? 1 : 0, pa = third == 2 ? 1 : 2;
     const size_t np = (size_t)len[pa] * len[pb];
     if (W.nn < np) {
-        if (W.nyq) (void)hipFree(W.nyq);
+        if (W.nyq) {
+            (void)hipFree(W.nyq);
+            ++W.freed;
+        }
         W.nyq = nullptr;
         W.nn = 0;
         const hipError_t e = hipMalloc((void**)&W.nyq, sizeof(float) * np);
@@ -691,7 +694,10 @@ int rot_run(RotWork& W, const float* src, float* vol, int nx, int ny, int nz, co
     int third = 0;
     if (planar_shears(P, planar, &third)) return run_planar(W, planar, third, src, vol, len, tw, st);
     if (W.wn < nv) {
-        if (W.w) (void)hipFree(W.w);
+        if (W.w) {
+            (void)hipFree(W.w);
+            ++W.freed;
+        }
         W.w = nullptr;
         W.wn = 0;
         hipError_t e = hipMalloc((void**)&W.w, sizeof(float2) * nv);

@@ -11,6 +11,7 @@ struct RotWork {
     size_t wn = 0;
     float* nyq = nullptr;             // planar rotations: Nyquist component along the third axis
     size_t nn = 0;
+    unsigned freed = 0;               // times w or nyq was given back
     std::map<int, float2*> tw;        // twiddle tables by line length
 };
 
