@@ -740,7 +740,7 @@ struct mset_recon {
     std::vector<float> prop_host;
     std::vector<mset_ctx*> tilts;
     std::vector<std::array<double, 3>> angles;
-    // the snapshot of every tilt's probe and positions, one after another
+    // the snapshot of every tilt's probe and positions, one after another, and their counts (empty: no snapshot)
     DevBuf<float2> probe_snap;
     DevBuf<float> pos_snap;
     std::vector<int> snap_npos;
@@ -1427,8 +1427,8 @@ int mset_recon_set_engine(mset_recon* r, int engine) {
     return MSET_OK;
 }
 
-// copies between the snapshot and the state, on the device
-static int snapshot_copy(mset_recon* r, bool save) {
+// copies between the snapshot and the state, on the device; had: the snapshot's positions per tilt
+static int snapshot_copy(mset_recon* r, bool save, const std::vector<int>& had) {
     const size_t n2 = (size_t)r->n * r->n, nv = n2 * r->nz;
     auto copy = [&](void* state, void* snap, size_t bytes) {
         return hipMemcpyAsync(save ? snap : state, save ? state : snap, bytes, hipMemcpyDeviceToDevice, r->stream);
@@ -1438,10 +1438,9 @@ static int snapshot_copy(mset_recon* r, bool save) {
     for (size_t j = 0; j < r->tilts.size(); ++j) {
         mset_ctx* c = r->tilts[j];
         HIPCHK(copy(c->probe.p, r->probe_snap.p + n2 * j, sizeof(float2) * n2));
-        const size_t had = r->snap_npos[j];       // positions when the snapshot was taken, at least c->npos
         HIPCHK(copy(c->x.p, r->pos_snap.p + off, sizeof(float) * c->npos));
-        HIPCHK(copy(c->y.p, r->pos_snap.p + off + had, sizeof(float) * c->npos));
-        off += 2 * had;
+        HIPCHK(copy(c->y.p, r->pos_snap.p + off + had[j], sizeof(float) * c->npos));
+        off += 2 * (size_t)had[j];
     }
     HIPCHK(hipStreamSynchronize(r->stream));
     return MSET_OK;
@@ -1449,24 +1448,29 @@ static int snapshot_copy(mset_recon* r, bool save) {
 
 int mset_recon_snapshot(mset_recon* r) {
     CHK(check_recon(r));
+    r->snap_npos.clear();                        // until every block is there and copied, there is no snapshot
     const size_t n2 = (size_t)r->n * r->n;
+    std::vector<int> npos;
+    size_t tot = 0;
+    for (const mset_ctx* c : r->tilts) {
+        npos.push_back(c->npos);
+        tot += c->npos;
+    }
     CHK(r->rec_snap.ensure(n2 * r->nz, "snapshot"));
     CHK(r->probe_snap.ensure(n2 * r->tilts.size(), "snapshot"));
-    size_t tot = 0;
-    for (const mset_ctx* c : r->tilts) tot += c->npos;
     CHK(r->pos_snap.ensure(2 * tot, "snapshot"));
-    r->snap_npos.clear();
-    for (const mset_ctx* c : r->tilts) r->snap_npos.push_back(c->npos);
-    return snapshot_copy(r, true);
+    CHK(snapshot_copy(r, true, npos));
+    r->snap_npos = npos;
+    return MSET_OK;
 }
 
 int mset_recon_restore(mset_recon* r) {
     CHK(check_recon(r));
-    if (!r->rec_snap.p) return fail(MSET_EINVAL, "no snapshot taken");
+    if (r->snap_npos.empty()) return fail(MSET_EINVAL, "no snapshot taken");
     for (size_t j = 0; j < r->tilts.size(); ++j)
         if (r->snap_npos[j] < r->tilts[j]->npos)
             return fail(MSET_EINVAL, "tilt " + std::to_string(j) + " has more positions than the snapshot");
-    return snapshot_copy(r, false);
+    return snapshot_copy(r, false, r->snap_npos);
 }
 
 int mset_recon_profile_enable(mset_recon* r, int enable) {
