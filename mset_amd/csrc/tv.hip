@@ -156,10 +156,13 @@ __global__ __launch_bounds__(256) void k_tv_iterate(int nx, int ny, int nz, cons
             // its remainder (Markstein, IBM J. Res. Dev. 34 (1990) 111): the arguments are normal and near 1, so the
             // scaling of a general division or square root is not needed, and the quotients share one reciprocal
             const float m = fmaxf(1.0f, q0 * q0 + q1 * q1 + q2 * q2);
-            const float rs = __builtin_amdgcn_rsqf(m);
-            float den = m * rs;
-            den = __builtin_fmaf(__builtin_fmaf(-den, den, m), 0.5f * rs, den);
-            const float r = __builtin_fmaf(__builtin_fmaf(-den, rs, 1.0f), rs, rs);
+            // beyond the float range (m infinite): r = 0, so finite q give 0 as their division by infinity does
+            const bool finite = m <= 3.402823466e38f;
+            const float mf = finite ? m : 1.0f;
+            const float rs = __builtin_amdgcn_rsqf(mf);
+            float den = mf * rs;
+            den = __builtin_fmaf(__builtin_fmaf(-den, den, mf), 0.5f * rs, den);
+            const float r = finite ? __builtin_fmaf(__builtin_fmaf(-den, rs, 1.0f), rs, rs) : 0.0f;
             auto quot = [&](float a) {
                 const float t = a * r;
                 return __builtin_fmaf(__builtin_fmaf(-den, t, a), r, t);
