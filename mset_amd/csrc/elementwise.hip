@@ -41,12 +41,12 @@ __global__ __launch_bounds__(256) void k_volume(float* V, const float* __restric
     if (p >= n2) return;
     for (int a = blockIdx.y; a < L; a += gridDim.y) {
         const int z0 = a * bin, z1 = min(z0 + bin, nz);
-        const float g = UPD ? s1 * G[(size_t)a * n2 + p] : 0.f;
+        const float g = UPD ? G[(size_t)a * n2 + p] : 0.f;
         float s = 0.f;
 #pragma unroll 4
         for (int z = z0; z < z1; ++z) {
             float v = V[(size_t)z * n2 + p];
-            if (UPD) V[(size_t)z * n2 + p] = v = v + g;
+            if (UPD) V[(size_t)z * n2 + p] = v = fmaf(s1, g, v);     // one rounding, as the line passes' step
             s += v;
         }
         if (TRANS) {
