@@ -29,39 +29,75 @@ __global__ void k_ingest(const float* __restrict__ M, float* __restrict__ out, i
     }
 }
 
-// Planes of a volume, one workgroup row per bin (blockIdx.y; the launch has one workgroup per 256 pixels and bin, so
-// an element costs no division: with 64-bit ones these kernels took 4.4 us on 24^3 voxels):
-//   UPD   V[z] += s1 G[a] for the slices z of bin a (the per-bin gradient replicated, STEP03_BACK.m:17-21)
-//   TRANS t_a = exp(1i * sigma * (sum_{z in bin a} V) * dx)  (STEP02_FORWARD_4D.m:12-20)
-// both: the object step of a position and the next one's transmission, the volume read once.
-template <bool UPD, bool TRANS>
-__global__ __launch_bounds__(256) void k_volume(float* V, const float* __restrict__ G, float2* __restrict__ T, int n2, int nz,
-                                                int bin, int L, float s1, int sset, float sigma, float dx) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= n2) return;
-    for (int a = blockIdx.y; a < L; a += gridDim.y) {
-        const int z0 = a * bin, z1 = min(z0 + bin, nz);
-        const float g = UPD ? G[(size_t)a * n2 + p] : 0.f;
-        float s = 0.f;
-#pragma unroll 4
-        for (int z = z0; z < z1; ++z) {
-            float v = V[(size_t)z * n2 + p];
-            if (UPD) V[(size_t)z * n2 + p] = v = fmaf(s1, g, v);     // one rounding, as the line passes' step
-            s += v;
-        }
-        if (TRANS) {
-            // STEP02_FORWARD_4D.m:18-19 rounds sigma * (sum * dx); STEP02_FORWARD_4D_SSET.m:9 (sigma * sum) * dx
-            const float ph = sset ? (sigma * s) * dx : sigma * (s * dx);
-            float sn, cs;
-            sincosf(ph, &sn, &cs);
-            T[(size_t)a * n2 + p] = make_float2(cs, sn);
+// Slices z0 .. z1 - 1 of a pixel, C of them loaded before the first is stored, summed in slice order; with UPD each takes
+// the object step first: V[z] += s1 g, one rounding, as in the line passes
+template <bool UPD, int C> __device__ __forceinline__ void slices(float* V, size_t n2, int& z, int z1, float s1, float g, float& s) {
+    for (; z + C <= z1; z += C) {
+        float v[C];
+#pragma unroll
+        for (int i = 0; i < C; ++i) v[i] = V[(z + i) * n2];
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+            if (UPD) V[(z + i) * n2] = v[i] = fmaf(s1, g, v[i]);
+            s += v[i];
         }
     }
 }
 
+// Planes of a volume (blockIdx.y: one workgroup per 256 pixels and bin or part of a bin, so an element costs no
+// division; with 64-bit ones these kernels took 4.4 us on 24^3 voxels).
+//
+// t_a = exp(1i * sigma * (sum_{z in bin a} V) * dx)  (STEP02_FORWARD_4D.m:12-20); with UPD the volume first takes the
+// object step, V[z] += s1 G[a] for the slices z of bin a (the per-bin gradient replicated, STEP03_BACK.m:17-21): a
+// position's step and the next one's transmission, the volume read once.  Up to 8 slices of a bin are in flight: with a
+// store after each load they were a chain of memory round trips, 10.0 -> 4.9 us for the single-slice operator (one bin)
+// on 64^3 voxels, 19.5 -> 7.8 us on 256 x 256 x 64.
+template <bool UPD>
+__global__ __launch_bounds__(256) void k_trans(float* V, const float* __restrict__ G, float2* __restrict__ T, int n2, int nz,
+                                               int bin, int L, float s1, int sset, float sigma, float dx) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= n2) return;
+    for (int a = blockIdx.y; a < L; a += gridDim.y) {
+        const int z1 = min(a * bin + bin, nz);
+        int z = a * bin;
+        const float g = UPD ? G[(size_t)a * n2 + p] : 0.f;
+        float s = 0.f;
+        slices<UPD, 8>(V + p, n2, z, z1, s1, g, s);
+        slices<UPD, 4>(V + p, n2, z, z1, s1, g, s);
+        slices<UPD, 2>(V + p, n2, z, z1, s1, g, s);
+        slices<UPD, 1>(V + p, n2, z, z1, s1, g, s);
+        // STEP02_FORWARD_4D.m:18-19 rounds sigma * (sum * dx); STEP02_FORWARD_4D_SSET.m:9 (sigma * sum) * dx
+        const float ph = sset ? (sigma * s) * dx : sigma * (s * dx);
+        float sn, cs;
+        sincosf(ph, &sn, &cs);
+        T[(size_t)a * n2 + p] = make_float2(cs, sn);
+    }
+}
+
+// The object step alone, UPDATE_SLICES slices of a bin per thread: a deep bin (the single-slice operator has one of the
+// whole depth) takes as many workgroups as its voxels ask for: 14.0 -> 3.6 us on 64^3 voxels, 19.6 -> 7.7 on
+// 256 x 256 x 64 against a thread per pixel of a bin; a thread per voxel reads G for each slice and takes 6.1 and 11.0 us,
+// 17.7 against 12.6 on 256 x 256 x 128 in bins of 4.
+constexpr int UPDATE_SLICES = 4;
+__global__ __launch_bounds__(256) void k_update_volume(float* V, const float* __restrict__ G, int n2, int nz, int bin, int parts,
+                                                       int rows, float s1) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= n2) return;
+    for (int r = blockIdx.y; r < rows; r += gridDim.y) {
+        const int a = r / parts;
+        int z = a * bin + (r - a * parts) * UPDATE_SLICES;
+        const int z1 = min(min(z + UPDATE_SLICES, a * bin + bin), nz);
+        const float g = G[(size_t)a * n2 + p];
+        float s = 0.f;
+        slices<true, 4>(V + p, n2, z, z1, s1, g, s);
+        slices<true, 2>(V + p, n2, z, z1, s1, g, s);
+        slices<true, 1>(V + p, n2, z, z1, s1, g, s);
+    }
+}
+
 // Transmission phases for the separable-propagator kernels, which form t = exp(i pi r) where they apply it
-// (half the bytes of a complex plane).  r is the f32 phase of k_volume, divided by pi and reduced to [-1, 1]
-// in double: t differs from k_volume's sincosf by about 1e-7.  Plane a goes to Tf in the
+// (half the bytes of a complex plane).  r is the f32 phase of k_trans, divided by pi and reduced to [-1, 1]
+// in double: t differs from k_trans's sincosf by about 1e-7.  Plane a goes to Tf in the
 // layout of the pass that applies it in the forward sweep (rows, [x][y], for even a; columns, [y][x], for
 // odd a) and, if Tb is given, to Tb in the layout of its adjoint pass (the other one).
 __global__ void k_trans_sep(const float* __restrict__ V, float* __restrict__ Tf, float* __restrict__ Tb, int n, int nz,
@@ -155,13 +191,14 @@ hipError_t launch_ingest_patterns(const float* M, float* sqrtM, int n, long long
 }
 
 namespace {
-dim3 volume_grid(int n2, int L) { return dim3((unsigned)((n2 + 255) / 256), (unsigned)(L < 65535 ? L : 65535)); }
+// 256 pixels by planes
+dim3 volume_grid(int n2, int planes) { return dim3((unsigned)((n2 + 255) / 256), (unsigned)(planes < 65535 ? planes : 65535)); }
 }  // namespace
 
 hipError_t launch_transmission(const float* V, float2* T, int n, int nz, int bin, int sset, float sigma, float dx,
                                hipStream_t st) {
     const int L = (nz + bin - 1) / bin;
-    hipLaunchKernelGGL((k_volume<false, true>), volume_grid(n * n, L), dim3(256), 0, st, const_cast<float*>(V), nullptr, T,
+    hipLaunchKernelGGL((k_trans<false>), volume_grid(n * n, L), dim3(256), 0, st, const_cast<float*>(V), nullptr, T,
                        n * n, nz, bin, L, 0.f, sset, sigma, dx);
     return hipGetLastError();
 }
@@ -206,11 +243,13 @@ hipError_t launch_update_volume(float* V, const float* G, int n, int nz, int bin
                                 int sset, float sigma, float dx) {
     const int L = (nz + bin - 1) / bin;
     if (trans)
-        hipLaunchKernelGGL((k_volume<true, true>), volume_grid(n * n, L), dim3(256), 0, st, V, G, trans, n * n, nz, bin, L, s1,
-                           sset, sigma, dx);
-    else
-        hipLaunchKernelGGL((k_volume<true, false>), volume_grid(n * n, L), dim3(256), 0, st, V, G, trans, n * n, nz, bin, L, s1,
-                           0, 0.f, 0.f);
+        hipLaunchKernelGGL((k_trans<true>), volume_grid(n * n, L), dim3(256), 0, st, V, G, trans, n * n, nz, bin, L, s1, sset,
+                           sigma, dx);
+    else {
+        const int parts = (bin + UPDATE_SLICES - 1) / UPDATE_SLICES;
+        hipLaunchKernelGGL(k_update_volume, volume_grid(n * n, L * parts), dim3(256), 0, st, V, G, n * n, nz, bin, parts, L * parts,
+                           s1);
+    }
     return hipGetLastError();
 }
 
