@@ -149,12 +149,14 @@ hipError_t launch_update_volume(float* V, const float* G, int n, int nz, int bin
 hipError_t launch_update_positions(float* x, float* y, const float* dpos, int npos, float s3, hipStream_t st);
 hipError_t launch_positivity(float* V, size_t n, hipStream_t st);
 
-// total-variation regulariser (tv.hip): two dual fields (3 volumes each) + f / lambda, reduction partials
+// total-variation regulariser (tv.hip): two dual fields (3 volumes each) + f / lambda, or one dual field and its
+// residual; reduction partials
 struct TvWork {
     float* P = nullptr;
     double* part = nullptr;
-    long long nv = 0;
+    size_t n = 0;              // elements of P
 };
+// scratch for a volume of nv elements: 7 volumes, or 4 where those do not fit
 int tv_ensure(TvWork& w, long long nv);
 void tv_release(TvWork& w);
 // u = TV_method(f, lambda, n_iter) on device volumes [nz][ny][nx] (u may equal f); err (nullable) gets

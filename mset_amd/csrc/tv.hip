@@ -4,7 +4,8 @@
 //   D = TV_div(P) - f / lambda
 //   P = TV_project(P + tau TV_del(D)), tau = 1/12
 // repeated n_iter times from P = 0, then u = f - lambda TV_div(P) and the error lambda sum |TV_del(u)|.
-// An iteration is one launch from one dual field to another (k_tv_iterate).
+// An iteration is one launch from one dual field to another (k_tv_iterate), on 7 volumes of scratch, or two launches in
+// place on 4 where 7 do not fit the device (k_tv_dual_residual, k_tv_project).
 // The dual field P is three float volumes (structure of arrays, so every stencil read is coalesced);
 // the operation order of each element follows TV_method.m so that single-precision results match a
 // MATLAB single run to rounding.  Volumes are [z][y][x] with MATLAB dims (x, y, z) = (1, 2, 3):
@@ -177,6 +178,36 @@ __global__ __launch_bounds__(256) void k_tv_iterate(int nx, int ny, int nz, cons
     }
 }
 
+// The same iteration in two launches, in place with the residual D stored: 4 volumes of scratch
+__global__ void k_tv_dual_residual(Grid3 g, const float* __restrict__ P0, const float* __restrict__ P1,
+                                   const float* __restrict__ P2, const float* __restrict__ f, float lambda,
+                                   float* __restrict__ D) {
+    const long long nv = (long long)g.nx * g.ny * g.nz;
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < nv; i += (long long)gridDim.x * blockDim.x) {
+        int x, y, z;
+        g.coords(i, x, y, z);
+        D[i] = tv_div(g, P0, P1, P2, x, y, z) - f[i] / lambda;
+    }
+}
+
+__global__ void k_tv_project(Grid3 g, float* __restrict__ P0, float* __restrict__ P1, float* __restrict__ P2,
+                             const float* __restrict__ D) {
+    const float tau = 1.0f / 12.0f;
+    const long long nv = (long long)g.nx * g.ny * g.nz;
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < nv; i += (long long)gridDim.x * blockDim.x) {
+        int x, y, z;
+        g.coords(i, x, y, z);
+        const float d = D[i];
+        const float q0 = P0[i] + tau * (D[g.at(x + 1 == g.nx ? 0 : x + 1, y, z)] - d);
+        const float q1 = P1[i] + tau * (D[g.at(x, y + 1 == g.ny ? 0 : y + 1, z)] - d);
+        const float q2 = P2[i] + tau * (D[g.at(x, y, z + 1 == g.nz ? 0 : z + 1)] - d);
+        const float den = sqrtf(fmaxf(1.0f, q0 * q0 + q1 * q1 + q2 * q2));
+        P0[i] = q0 / den;
+        P1[i] = q1 / den;
+        P2[i] = q2 / den;
+    }
+}
+
 __global__ void k_tv_output(Grid3 g, const float* __restrict__ P0, const float* __restrict__ P1,
                             const float* __restrict__ P2, const float* f, float lambda, float* u) {
     const long long nv = (long long)g.nx * g.ny * g.nz;
@@ -243,16 +274,21 @@ dim3 grid_of(long long n) {
 }  // namespace
 
 int tv_ensure(TvWork& w, long long nv) {
-    if (w.nv >= nv && w.P) return 0;
-    if (w.P) (void)hipFree(w.P);
-    if (w.part) (void)hipFree(w.part);
-    w.P = nullptr;
-    w.part = nullptr;
-    w.nv = 0;
-    if (hipMalloc((void**)&w.P, sizeof(float) * 7 * (size_t)nv) != hipSuccess) return -1;
-    if (hipMalloc((void**)&w.part, sizeof(double) * RED_BLOCKS) != hipSuccess) return -1;
-    w.nv = nv;
-    return 0;
+    if (w.P && w.n >= 7 * (size_t)nv) return 0;
+    tv_release(w);
+    if (hipMalloc((void**)&w.part, sizeof(double) * RED_BLOCKS) != hipSuccess) {
+        w.part = nullptr;
+        return -1;
+    }
+    for (const size_t volumes : {7, 4}) {
+        if (hipMalloc((void**)&w.P, sizeof(float) * volumes * (size_t)nv) == hipSuccess) {
+            w.n = volumes * (size_t)nv;
+            return 0;
+        }
+        (void)hipGetLastError();                         // not the next launch's error
+        w.P = nullptr;
+    }
+    return -1;
 }
 
 void tv_release(TvWork& w) {
@@ -260,33 +296,43 @@ void tv_release(TvWork& w) {
     if (w.part) (void)hipFree(w.part);
     w.P = nullptr;
     w.part = nullptr;
-    w.nv = 0;
+    w.n = 0;
 }
 
 hipError_t tv_run(TvWork& w, const float* f, float* u, int nx, int ny, int nz, float lambda, int n_iter, double* err,
                   hipStream_t st) {
     const Grid3 g{nx, ny, nz};
     const long long nv = (long long)nx * ny * nz;
-    // two dual fields and f / lambda
-    float *P = w.P, *Q = w.P + 3 * nv, *q = w.P + 6 * nv;
+    float* P = w.P;
     const dim3 gr = grid_of(nv), bl(RED_THREADS);
     hipError_t e = launch_fill(P, sizeof(float) * 3 * (size_t)nv, st);   // P = 0
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_tv_scale, gr, bl, 0, st, f, nv, lambda, q);
-    const bool wide = nx % 4 == 0;                       // rows of whole float4s
-    const long long items = wide ? nv / 4 : nv;
-    const bool narrow_index = nv < (1LL << 30);          // 32-bit byte offsets
-    for (int it = 0; it < n_iter; ++it) {
-        const dim3 gi = grid_of(items);
-        if (wide && narrow_index)
-            hipLaunchKernelGGL((k_tv_iterate<4, unsigned>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (unsigned)items);
-        else if (wide)
-            hipLaunchKernelGGL((k_tv_iterate<4, unsigned long long>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (unsigned long long)items);
-        else if (narrow_index)
-            hipLaunchKernelGGL((k_tv_iterate<1, unsigned>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (unsigned)items);
-        else
-            hipLaunchKernelGGL((k_tv_iterate<1, unsigned long long>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (unsigned long long)items);
-        std::swap(P, Q);
+    if (w.n < 7 * (size_t)nv) {
+        float* D = w.P + 3 * nv;
+        for (int it = 0; it < n_iter; ++it) {
+            hipLaunchKernelGGL(k_tv_dual_residual, gr, bl, 0, st, g, P, P + nv, P + 2 * nv, f, lambda, D);
+            hipLaunchKernelGGL(k_tv_project, gr, bl, 0, st, g, P, P + nv, P + 2 * nv, D);
+        }
+    } else {
+        // two dual fields and f / lambda
+        float *Q = w.P + 3 * nv, *q = w.P + 6 * nv;
+        hipLaunchKernelGGL(k_tv_scale, gr, bl, 0, st, f, nv, lambda, q);
+        const bool wide = nx % 4 == 0;                   // rows of whole float4s
+        const long long items = wide ? nv / 4 : nv;
+        const bool narrow_index = nv < (1LL << 30);      // 32-bit byte offsets
+        using U64 = unsigned long long;
+        for (int it = 0; it < n_iter; ++it) {
+            const dim3 gi = grid_of(items);
+            if (wide && narrow_index)
+                hipLaunchKernelGGL((k_tv_iterate<4, unsigned>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (unsigned)items);
+            else if (wide)
+                hipLaunchKernelGGL((k_tv_iterate<4, U64>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (U64)items);
+            else if (narrow_index)
+                hipLaunchKernelGGL((k_tv_iterate<1, unsigned>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (unsigned)items);
+            else
+                hipLaunchKernelGGL((k_tv_iterate<1, U64>), gi, bl, 0, st, nx, ny, nz, P, q, Q, (U64)items);
+            std::swap(P, Q);
+        }
     }
     const float *P0 = P, *P1 = P + nv, *P2 = P + 2 * nv;
     hipLaunchKernelGGL(k_tv_output, gr, bl, 0, st, g, P0, P1, P2, f, lambda, u);

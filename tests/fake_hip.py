@@ -73,3 +73,46 @@ def run(tmp, body):
     r = subprocess.run([sys.executable, '-c', code], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
     return r.stdout
+
+
+FAIL_SOURCE = '''
+#include <dlfcn.h>
+#include <stddef.h>
+static size_t size;
+static int count;
+void fail_malloc(size_t n) { size = n; }
+int failed(void) { return count; }
+int hipMalloc(void** p, size_t n) {
+    static int (*real)(void**, size_t);
+    if (!real) real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
+    if (size && n == size) {
+        *p = 0;
+        ++count;
+        return 2;            /* hipErrorOutOfMemory */
+    }
+    return real(p, n);
+}
+'''
+
+FAIL_PRELUDE = '''
+import ctypes as C
+import sys
+shim = C.CDLL(%(so)r, mode=C.RTLD_GLOBAL)
+shim.fail_malloc.argtypes = [C.c_size_t]
+fail_malloc, failed = shim.fail_malloc, shim.failed
+sys.path.insert(0, %(root)r)
+import numpy as np
+from mset_amd import lib
+'''
+
+
+def run_failing_malloc(tmp, body):
+    """Runs `body` in a child process on the real runtime, where device allocations of exactly fail_malloc(n) bytes
+    report that the device is out of memory; failed() counts them."""
+    so, c = os.path.join(str(tmp), 'libfail_malloc.so'), os.path.join(str(tmp), 'fail_malloc.c')
+    with open(c, 'w') as fh:
+        fh.write(FAIL_SOURCE)
+    subprocess.run(['gcc', '-O1', '-shared', '-fPIC', c, '-o', so, '-ldl'], check=True)
+    code = FAIL_PRELUDE % dict(so=so, root=ROOT) + textwrap.dedent(body)
+    r = subprocess.run([sys.executable, '-c', code], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]

@@ -44,3 +44,29 @@ def test_large_arguments_stay_finite(nx, size):
     assert np.isfinite(ref).all() and np.isfinite(out).all()
     # every P is within [-1, 1], its 6 terms rounded to float32 per iteration; u adds the rounding of the voxel
     assert (np.abs(out.astype(np.float64) - ref) <= 6 * 6 * 2.0 ** -22 + 2.0 ** -22 * np.abs(ref)).all()
+
+
+# rows of whole float4s and others, odd and even iteration counts
+@pytest.mark.parametrize('shape,iters', [((5, 6, 8), 6), ((9, 17, 33), 11), ((16, 24, 20), 0), ((1, 1, 4), 3)])
+def test_small_scratch_gives_the_same(tmp_path, shape, iters):
+    """the two-launch iteration on 4 volumes of scratch against the one-launch one on 7 and TV_method"""
+    from oracle import oracle as O
+    from tests.conftest import rel
+    from tests.fake_hip import run_failing_malloc
+    v = np.random.default_rng(sum(shape)).uniform(0, 3, shape).astype(np.float32)
+    np.save(tmp_path / 'v.npy', v)
+    print('case: tv small scratch', shape, iters, flush=True)
+    run_failing_malloc(tmp_path, '''
+        v = np.load(%r)
+        with lib.Context(0) as ctx:
+            whole, e = ctx.tv(v, 0.25, %d)
+        fail_malloc(7 * v.size * 4)
+        with lib.Context(0) as ctx:
+            out, e2 = ctx.tv(v, 0.25, %d)
+        assert failed() == 1
+        np.savez(%r, whole=whole, out=out, e=[e, e2])
+    ''' % (str(tmp_path / 'v.npy'), iters, iters, str(tmp_path / 'o.npz')))
+    o = np.load(tmp_path / 'o.npz')
+    ref, rerr = O.tv(v, 0.25, iters)
+    for u, e in ((o['whole'], o['e'][0]), (o['out'], o['e'][1])):
+        assert rel(u, ref) < 1e-5 and abs(e - rerr) <= 1e-4 * abs(rerr) + 1e-5
