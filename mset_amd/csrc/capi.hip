@@ -49,6 +49,10 @@ int fail(int code, const std::string& msg) {
         if (r_ != MSET_OK) return r_;     \
     } while (0)
 
+// Frees what the workspace of the call in progress on this thread keeps between calls only to save allocations (the TV
+// scratch and the host-to-host volume, neither in use while a DevBuf allocates); false if there was nothing
+bool give_back_kept();
+
 template <typename T> struct DevBuf {
     T* p = nullptr;
     size_t n = 0;
@@ -70,7 +74,9 @@ template <typename T> struct DevBuf {
         release();
         if (count == 0) return MSET_OK;
         hipError_t e = hipMalloc((void**)&p, count * sizeof(T));
+        if (e != hipSuccess && give_back_kept()) e = hipMalloc((void**)&p, count * sizeof(T));
         if (e != hipSuccess) {
+            (void)hipGetLastError();                     // not the next launch's error
             p = nullptr;
             return fail(MSET_ENOMEM, std::string("hipMalloc ") + what + ": " + hipGetErrorString(e));
         }
@@ -109,6 +115,17 @@ struct Workspace {
         tv_release(tv);
     }
 };
+
+thread_local std::weak_ptr<Workspace> g_call_ws;   // set by the checks that every entry point begins with
+
+bool give_back_kept() {
+    const std::shared_ptr<Workspace> W = g_call_ws.lock();
+    if (!W || (!W->tv.P && !W->io.p)) return false;
+    (void)hipGetLastError();                       // of the allocation that did not fit
+    tv_release(W->tv);
+    W->io.release();
+    return true;
+}
 
 }  // namespace
 
@@ -214,6 +231,7 @@ unsigned char* scratch_on(int device) {
 int check_ctx(mset_ctx* c) {
     if (!c) return fail(MSET_EINVAL, "null context");
     HIPCHK(hipSetDevice(c->device));
+    g_call_ws = c->ws;
     return MSET_OK;
 }
 
@@ -707,6 +725,17 @@ int upload_impl(mset_ctx* c, const mset_params* p, const float* RVol, const floa
     return MSET_OK;
 }
 
+// rot_run; its buffers are allocated before its first launch, and where they do not fit the TV scratch makes room
+int rotate_or_give_back(mset_ctx* c, const float* src, float* vol, int nx, int ny, int nz, const double* R, double step) {
+    int r = rot_run(c->ws->rot, src, vol, nx, ny, nz, R, step, c->stream);
+    if (r == MSET_ENOMEM && c->ws->tv.P) {
+        (void)hipGetLastError();
+        tv_release(c->ws->tv);
+        r = rot_run(c->ws->rot, src, vol, nx, ny, nz, R, step, c->stream);
+    }
+    return r == MSET_OK ? r : fail(r, rot_last_error());
+}
+
 // vol = rotation of src (src may be vol)
 int rotate_volume(mset_ctx* c, const float* src, float* vol, const double* v1, const double* v2, const double* v3,
                   const double* ang, bool inverse) {
@@ -719,9 +748,7 @@ int rotate_volume(mset_ctx* c, const float* src, float* vol, const double* v1, c
     if (!rot_size_supported(c->n) || !rot_size_supported(c->nz))
         return fail(MSET_EUNSUPPORTED, "rotation line length not built");
     Timed t(c, "rotate");
-    const int r = rot_run(c->ws->rot, src, vol, c->n, c->n, c->nz, R, 11.0, c->stream);
-    if (r != MSET_OK) return fail(r, rot_last_error());
-    return MSET_OK;
+    return rotate_or_give_back(c, src, vol, c->n, c->n, c->nz, R, 11.0);
 }
 
 }  // namespace
@@ -767,6 +794,7 @@ void drop_graph(mset_recon* r) {
 int check_recon(mset_recon* r) {
     if (!r) return fail(MSET_EINVAL, "null reconstruction");
     HIPCHK(hipSetDevice(r->device));
+    g_call_ws = r->ws;
     for (size_t j = 0; j < r->tilts.size(); ++j)
         if (!r->tilts[j] || !r->tilts[j]->uploaded)
             return fail(MSET_EINVAL, "tilt " + std::to_string(j) + " has no data (call mset_recon_set_tilt)");
@@ -1069,8 +1097,7 @@ int mset_rotate(mset_ctx* c, const float* in, float* out, int nx, int ny, int nz
     HIPCHK(hipMemcpyAsync(buf.p, in, sizeof(float) * nv, hipMemcpyHostToDevice, c->stream));
     {
         Timed t(c, "rotate");
-        const int r = rot_run(c->ws->rot, buf.p, buf.p, nx, ny, nz, R, step, c->stream);
-        if (r != MSET_OK) return fail(r, rot_last_error());
+        CHK(rotate_or_give_back(c, buf.p, buf.p, nx, ny, nz, R, step));
     }
     HIPCHK(hipMemcpyAsync(out, buf.p, sizeof(float) * nv, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1214,6 +1241,7 @@ int mset_recon_set_tilt(mset_recon* r, int j, const double* angles, const float*
                         int num_scan_pos, const float* xlist, const float* ylist, const float* measured) {
     if (!r) return fail(MSET_EINVAL, "null reconstruction");
     HIPCHK(hipSetDevice(r->device));
+    g_call_ws = r->ws;
     if (j < 0 || j >= (int)r->tilts.size()) return fail(MSET_EINVAL, "tilt index out of range");
     if (!angles) return fail(MSET_EINVAL, "null angles");
     drop_graph(r);

@@ -687,7 +687,8 @@ int rot_run(RotWork& W, const float* src, float* vol, int nx, int ny, int nz, co
     for (int a = 0; a < 3; ++a) {
         hipError_t e = hipSuccess;
         tw[a] = twiddle_table(W, len[a], st, e);
-        if (!tw[a]) return rfail(MSET_EDEVICE, std::string("twiddles: ") + hipGetErrorString(e));
+        if (!tw[a])
+            return rfail(e == hipErrorOutOfMemory ? MSET_ENOMEM : MSET_EDEVICE, std::string("twiddles: ") + hipGetErrorString(e));
     }
     const ShearPlan P = plan_rotation(R, rot_step_init);
     std::vector<PlanarShear> planar;

@@ -51,12 +51,13 @@ int fake_stale_replays() { return g_stale_replays; }
 size_t fake_bytes() { return g_bytes; }
 size_t fake_peak() { return g_peak; }
 void fake_fail_malloc(size_t bytes) { g_fail = bytes; }   // allocations of exactly this size fail (0: none)
+void fake_device_memory(size_t bytes) { g_total = bytes; }   // allocations beyond it fail
 void fake_occupancy(const char* part, int per_cu) { g_occ[part] = per_cu; }
 
 // ---- the runtime
 hipError_t hipMalloc(void** p, size_t n) {
     *p = nullptr;
-    if (g_fail && n == g_fail) return hipErrorOutOfMemory;
+    if ((g_fail && n == g_fail) || g_bytes + n > g_total) return hipErrorOutOfMemory;
     *p = calloc(1, n ? n : 1);
     g_live[*p] = n;
     g_bytes += n;
