@@ -336,14 +336,13 @@ int shape_for(const mset_ctx* c, int waves, bool fixed) {
 }
 
 // workgroups of the batched kernel of a workgroup shape the device keeps resident at once (1 per CU at
-// N = 128 in the default shape); by default the shape of the last batched call
+// N = 128 in the default shape)
 int device_slots(mset_ctx* c, int shape) {
     int per_cu = 1;
     const hipError_t e = shape == SHAPE_SEP ? occupancy_sep(c->n, false, &per_cu) : occupancy_batch(c->n, shape, &per_cu);
     if (e != hipSuccess || per_cu < 1) per_cu = 1;
     return c->cus * per_cu;
 }
-int device_slots(mset_ctx* c) { return device_slots(c, c->ws->shape); }
 
 // the persistent grid of the batched kernels: the resident workgroups, capped by the slot limit and the
 // positions
@@ -353,13 +352,11 @@ int batch_slots(mset_ctx* c, int shape) {
     if (s > c->npos) s = c->npos;
     return s < 1 ? 1 : s;
 }
-int batch_slots(mset_ctx* c) { return batch_slots(c, c->ws->shape); }
 
 // Gradient slabs of the context's batched launches: position p of a launch adds to slab p % S.  S depends
 // on the device, the workgroup shape and the positions only, never on the slot limit, so capping the grid
 // leaves every sum (and so every result) bitwise unchanged.
 int grad_slabs(mset_ctx* c, int shape) { return std::max(1, std::min(device_slots(c, shape), c->npos)); }
-int grad_slabs(mset_ctx* c) { return grad_slabs(c, c->ws->shape); }
 
 // The workgroup shape of a batched launch.  A launch with at most one position per CU takes the large workgroup
 // where the default one is sized for several positions per CU: with stored waves at 48 (202 -> 150 us at 256
@@ -384,14 +381,15 @@ int launch_grid(int want, int count, int S) {
     return g;
 }
 
-int ensure_fixed_buffers(mset_ctx* c) {
+// slots: the grid of the launch that follows
+int ensure_fixed_buffers(mset_ctx* c, int slots) {
     Workspace& W = *c->ws;
     // complex planes, or (separable routine) f32 phases in the forward and the adjoint layouts: L planes
     // either way
     CHK(W.trans.ensure(plane(c) * c->L, "transmission"));
     CHK(W.probeF.ensure(plane(c), "probe spectrum"));
     // the position kernels of the largest planes keep the plane in global memory: 2 planes per slot
-    if (plane_in_global(c->n)) CHK(W.planes.ensure((size_t)batch_slots(c) * 2 * plane(c), "plane buffers"));
+    if (plane_in_global(c->n)) CHK(W.planes.ensure((size_t)slots * 2 * plane(c), "plane buffers"));
     return MSET_OK;
 }
 
@@ -437,12 +435,12 @@ int ensure_batch_buffers(mset_ctx* c, bool fixed) {
     CHK(resolve_exit_waves(c, batch_slots(c, 0), &wv));
     W.waves = wv;
     W.shape = shape_for(c, wv, fixed);
-    const int s = batch_slots(c);
-    CHK(ensure_fixed_buffers(c));
+    const int s = batch_slots(c, W.shape);
+    CHK(ensure_fixed_buffers(c, s));
     const int save_planes = wave_planes(c, wv);
     CHK(W.save.ensure((size_t)s * save_planes * plane(c), "save waves"));
     W.slot_bytes = plane(c) * (save_planes * sizeof(float2) + (size_t)planes(c) * sizeof(float));
-    const int S = grad_slabs(c);
+    const int S = grad_slabs(c, W.shape);
     CHK(W.gslab.ensure((size_t)S * c->L * plane(c), "gradient slabs"));
     CHK(W.pslab.ensure((size_t)S * plane(c), "probe slabs"));
     CHK(W.G.ensure((size_t)c->L * plane(c), "gradient"));
@@ -454,8 +452,8 @@ int ensure_batch_buffers(mset_ctx* c, bool fixed) {
 
 // transmission planes + fftn(probe) for the fixed-state kernels; sep: 1 = forward layouts of the separable
 // kernels, 2 = forward and adjoint layouts
-int prepare_fixed(mset_ctx* c, int sep = 0) {
-    CHK(ensure_fixed_buffers(c));
+int prepare_fixed(mset_ctx* c, int slots, int sep = 0) {
+    CHK(ensure_fixed_buffers(c, slots));
     if (sep)
         HIPCHK(launch_transmission_sep(c->V.p, (float*)c->ws->trans.p, sep == 2 ? (float*)c->ws->trans.p + plane(c) * c->L : nullptr,
                                        c->n, c->nz, binning(c), c->p.sigma, c->p.potential_pixelsize, c->stream));
@@ -501,7 +499,7 @@ int issue_plain(mset_ctx* c) {
         }
         return MSET_OK;
     }
-    CHK(ensure_fixed_buffers(c));
+    CHK(ensure_fixed_buffers(c, 1));
     CHK(c->ws->gslab.ensure((size_t)c->L * plane(c), "gradient planes"));
     PosArgs A = base_args(c);
     const float s1 = c->p.step_size[0];
@@ -534,15 +532,16 @@ int fwd_slots(const mset_ctx* c) {
 
 int issue_fwd(mset_ctx* c, float* inten) {
     const bool sep = sep_fwd(c);
-    CHK(prepare_fixed(c, sep ? 1 : 0));
+    const int grid = sep_fwd_lines(c) ? std::min(fwd_slots(c), c->npos) : batch_slots(c, 0);   // the kernels' own shape
+    CHK(prepare_fixed(c, grid, sep ? 1 : 0));
     PosArgs A = base_args(c);
     A.sep = sep ? 1 : 0;
     A.first = 0;
     A.count = c->npos;
     A.inten = inten;
     Timed t(c, "position_fwd");
-    if (sep_fwd_lines(c)) HIPCHK(launch_sep_fwd(c->n, A, std::min(fwd_slots(c), c->npos), false, c->stream));
-    else HIPCHK(launch_fwd(c->n, A, plane_in_global(c->n) ? batch_slots(c) : batch_slots(c, 0), fwd_shape(c, c->npos), c->stream));
+    if (sep_fwd_lines(c)) HIPCHK(launch_sep_fwd(c->n, A, grid, false, c->stream));
+    else HIPCHK(launch_fwd(c->n, A, grid, fwd_shape(c, c->npos), c->stream));
     return MSET_OK;
 }
 
@@ -552,9 +551,9 @@ int issue_fwd(mset_ctx* c, float* inten) {
 int issue_grad(mset_ctx* c, int first, int count, bool apply, int want) {
     CHK(ensure_batch_buffers(c, !apply));
     const bool sep = sep_batch(c);
-    CHK(prepare_fixed(c, sep ? 2 : 0));
+    CHK(prepare_fixed(c, c->slots, sep ? 2 : 0));
     Workspace& W = *c->ws;
-    const int S = grad_slabs(c);
+    const int S = grad_slabs(c, W.shape);
     const int grid = launch_grid(c->slots, count, S);
     const int used = std::min(count, S);                 // slabs written by this launch
     PosArgs A = base_args(c);
@@ -1021,7 +1020,7 @@ int mset_waves(mset_ctx* c, int k, float* waves_out) {
     if (k < 0 || k >= c->npos || !waves_out) return fail(MSET_EINVAL, "bad position index or null output");
     CHK(set_method(c, MSET_METHOD_MSET));
     CHK(ensure_batch_buffers(c, true));
-    CHK(prepare_fixed(c));
+    CHK(prepare_fixed(c, 1));
     // every plane's wave is read back: the store layout, in slot 0
     CHK(c->ws->save.ensure((size_t)(c->L + 2) * plane(c), "save waves"));
     PosArgs A = base_args(c);

@@ -19,3 +19,29 @@ def test_object_step_has_a_thread_per_4_voxels(tmp, n, nz, binning, method):
         (name, gx, gy, threads, _), = launches('update_volume') or launches('k_volume<true')
         assert 4 * gx * gy * threads >= %d, (name, gx, gy, threads)
     ''' % (n, nz, binning, method, n * n * nz))
+
+
+@pytest.mark.parametrize('engine', ['AUTO', 'ALT_SHAPE', 'GENERAL'])
+def test_forward_grid_does_not_depend_on_earlier_calls(tmp, engine):
+    """the error pass of one position size after batched calls of another, and after another engine's"""
+    fake_hip.run(tmp, '''
+        fake.fake_occupancy(b'k_batch<256, 1', 3)
+        def grid(before):
+            ctx = lib.Context(0)
+            for n, e in before:
+                upload(ctx, n, 2, 5)
+                ctx.set_engine(e)
+                ctx.run_batched(5)
+            upload(ctx, 256, 2, 700)
+            ctx.set_engine(lib.ENGINE_%s)
+            fake.fake_reset()
+            ctx.error_resident()
+            (name, gx, _, threads, _), = launches('k_fwd<256')
+            planes = fake.fake_bytes()
+            ctx.close()
+            return name, gx, threads
+        fresh = grid(())
+        assert fresh[1] == 512                   # two workgroups on each of 256 CUs
+        for before in (((64, 0),), ((24, 0),), ((64, 2),), ((256, 2),), ((256, 1), (48, 0)), ((256, 0),)):
+            assert grid(before) == fresh, before
+    ''' % engine)
