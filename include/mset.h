@@ -249,8 +249,10 @@ int mset_host_free(void* ptr);
 /* ---- device capacity (admission control for several reconstructions on one device) ------------- */
 /* Free and total device memory in bytes. */
 int mset_device_memory(int device, size_t* free_bytes, size_t* total_bytes);
-/* Workgroups the batched position kernel keeps resident for plane size n: the number of per-slot
- * workspaces (saved waves, gradient slabs) a context allocates. */
+/* Workgroups the batched position kernels keep resident for plane size n, in the default engine: the largest
+ * number of per-slot workspaces (saved waves, gradient slabs) a context allocates.  Below 128 two routines share
+ * the work (MSET_ENGINE_AUTO) and this is the larger of their numbers; a call whose routine keeps fewer resident
+ * allocates fewer. */
 int mset_batch_slots(int device, int n, int* slots);
 
 /* ---- instrumentation -------------------------------------------------------------------------- */

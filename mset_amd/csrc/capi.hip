@@ -1140,8 +1140,12 @@ int mset_batch_slots(int device, int n, int* slots) {
     HIPCHK(hipSetDevice(device));
     hipDeviceProp_t prop;
     HIPCHK(hipGetDeviceProperties(&prop, device));
-    int per_cu = 1;
+    // the routines a batched call may run: the general one (mset_grad, the exact pairing, other propagators) and, below
+    // 128, the on-chip separable one (updates)
+    int per_cu = 1, per_cu_sep = 1;
     HIPCHK(occupancy_batch(n, 0, &per_cu));
+    if (n < 128) HIPCHK(occupancy_sep(n, false, &per_cu_sep));
+    per_cu = std::max(per_cu, per_cu_sep);
     *slots = prop.multiProcessorCount * (per_cu < 1 ? 1 : per_cu);
     return MSET_OK;
 }

@@ -45,3 +45,42 @@ def test_forward_grid_does_not_depend_on_earlier_calls(tmp, engine):
         for before in (((64, 0),), ((24, 0),), ((64, 2),), ((256, 2),), ((256, 1), (48, 0)), ((256, 0),)):
             assert grid(before) == fresh, before
     ''' % engine)
+
+
+# the general routine keeping fewer workgroups than the separable one, and more
+@pytest.mark.parametrize('n,general,separable', [(24, 5, 6), (16, 16, 19), (64, 3, 2), (96, 1, 1), (128, 1, 9)])
+def test_batch_slots_covers_the_kernels_of_a_batched_call(tmp, n, general, separable):
+    fake_hip.run(tmp, '''
+        n, g, s = %d, %d, %d
+        fake.fake_occupancy(b'k_batch<%%d, 0' %% n, g)
+        fake.fake_occupancy(b'k_sep_batch<%%d' %% n, s)
+        slots = lib.batch_slots(n)
+        per_cu = max(g, s) if n < 128 else g
+        assert slots == 256 * per_cu, slots
+        ctx = lib.Context(0)
+        npos = 256 * max(g, s) + 3 if n < 32 else 600
+        for separable in (True, False):
+            upload(ctx, n, 2, npos, separable=separable)
+            fake.fake_reset()
+            ctx.run_batched(npos)
+            (name, gx, _, _, _), = launches('k_sep_batch') + launches('k_batch')
+            assert gx <= slots, (name, gx, slots)
+            if npos > slots:
+                assert gx == 256 * (s if 'sep' in name else g), (name, gx)
+    ''' % (n, general, separable))
+
+
+@pytest.mark.parametrize('P,vol', [(32, 16), (64, 32), (128, 32), (256, 16)])
+def test_serving_footprint_covers_what_a_job_allocates(tmp, P, vol):
+    fake_hip.run(tmp, '''
+        from mset_amd import serve
+        fake.fake_occupancy(b'k_batch<', 2)
+        fake.fake_occupancy(b'k_sep_batch<', 5)
+        spec = serve.JobSpec(job_id=0, vol=%d, P=%d, tilts=[0.0, 10.0], scan=16, seed=1)
+        fake.fake_reset()
+        r = serve.make_recon(spec)
+        for _ in range(2):
+            r.iterate(1, 128, True, True)
+        r.snapshot()
+        assert fake.fake_peak() <= serve.footprint_bytes(spec, lib.batch_slots(spec.P)), (fake.fake_peak(), serve.footprint_bytes(spec, lib.batch_slots(spec.P)))
+    ''' % (vol, P))
