@@ -5,6 +5,14 @@
 
 namespace mset {
 
+namespace {
+// Cfg of the alternative shape; at 16 the default workgroup of one wave is the faster one with every routine
+template <int N> constexpr int ALT = N == 16 ? 0 : 1;
+// whether it applies a separable propagator as its 1D factors: at 32 they cost a workgroup per CU (1400 positions x 12
+// planes 234 us with them, 188 without)
+template <int N> constexpr bool ALT_PFAC = N != 32;
+}  // namespace
+
 hipError_t launch_batch_variant(int n, const PosArgs& A, int grid, int shape, hipStream_t st);
 
 hipError_t launch_batch(int n, const PosArgs& A, int grid, int shape, hipStream_t st) {
@@ -23,9 +31,9 @@ hipError_t launch_batch(int n, const PosArgs& A, int grid, int shape, hipStream_
         if (A.pfac && !A.sset) hipLaunchKernelGGL((k_batch<48, 2, WAVES_STORE, false, true>), dim3(grid), dim3(Cfg<48, 2>::NT), 0, st, A);
         else hipLaunchKernelGGL((k_batch<48, 2, WAVES_STORE, false>), dim3(grid), dim3(Cfg<48, 2>::NT), 0, st, A);
     } else if (shape && A.pfac && n < 128 && !A.sset) {
-        MSET_DISPATCH_SMALL(n, hipLaunchKernelGGL((k_batch<NN, 1, WAVES_STORE, false, true>), dim3(grid), dim3(Cfg<NN, 1>::NT), 0, st, A))
+        MSET_DISPATCH_SMALL(n, hipLaunchKernelGGL((k_batch<NN, ALT<NN>, WAVES_STORE, false, ALT_PFAC<NN>>), dim3(grid), dim3(Cfg<NN, ALT<NN>>::NT), 0, st, A))
     } else if (shape) {
-        MSET_DISPATCH(n, hipLaunchKernelGGL((k_batch<NN, 1, WAVES_STORE, false>), dim3(grid), dim3(Cfg<NN, 1>::NT), 0, st, A))
+        MSET_DISPATCH(n, hipLaunchKernelGGL((k_batch<NN, ALT<NN>, WAVES_STORE, false>), dim3(grid), dim3(Cfg<NN, ALT<NN>>::NT), 0, st, A))
     } else if (A.pfac && n != 256 && !A.sset) {
         MSET_DISPATCH_SMALL(n, hipLaunchKernelGGL((k_batch<NN, 0, WAVES_STORE, false, true>), dim3(grid), dim3(Cfg<NN>::NT), 0, st, A))
     } else MSET_DISPATCH(n, hipLaunchKernelGGL((k_batch<NN, 0, WAVES_STORE, false>), dim3(grid), dim3(Cfg<NN>::NT), 0, st, A));
@@ -34,7 +42,7 @@ hipError_t launch_batch(int n, const PosArgs& A, int grid, int shape, hipStream_
 
 hipError_t occupancy_batch(int n, int shape, int* blocks_per_cu) {
     if (shape)
-        MSET_DISPATCH(n, return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, (k_batch<NN, 1, WAVES_STORE, false>), Cfg<NN, 1>::NT, 0));
+        MSET_DISPATCH(n, return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, (k_batch<NN, ALT<NN>, WAVES_STORE, false>), Cfg<NN, ALT<NN>>::NT, 0));
     MSET_DISPATCH(n, return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, (k_batch<NN, 0, WAVES_STORE, false>), Cfg<NN>::NT, 0));
     return hipSuccess;
 }

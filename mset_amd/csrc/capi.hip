@@ -364,8 +364,12 @@ int grad_slabs(mset_ctx* c, int shape) { return std::max(1, std::min(device_slot
 // with stored or checkpointed waves (a tilt's last mini-batch, 15-20 % shorter at 64-256 positions).  The line
 // transforms, operand order and slab assignment are the default shape's, so the gradient slabs are the same bit
 // for bit; the workgroup sums (loss, position terms) add their terms in another order.
+// The alternative shape at 64 is the other way round, a small workgroup that pays from two positions per CU on (64 x 64 x 12
+// planes, 256 positions: 296 us, and 187 in the default shape), so a short launch takes the default one.
 int batch_shape(const mset_ctx* c, int shape, bool sep, int waves, int count) {
-    if (shape != 0 || count > c->cus) return shape;
+    if (count > c->cus) return shape;
+    if (c->n == 64 && shape == 1) return 0;
+    if (shape != 0) return shape;
     if (c->n == 48 && waves == WAVES_STORE) return 2;
     return c->n == 256 && sep && (waves == WAVES_STORE || waves == WAVES_CHECKPOINT) ? 2 : 0;
 }

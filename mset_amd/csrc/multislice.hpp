@@ -50,10 +50,12 @@ namespace mset {
 // the better one once positions share a CU (665 against 721 us at 1400) and the large one, SH = 2, below that
 // (202 -> 150 us at 256).  These kernels serve what the on-chip separable routine (sep_lines.hpp) does not: mset_grad,
 // the exact pairing, recomputed and checkpointed waves, other propagators, the single-slice operator.
-// SH = 1: the alternative shape of the batched kernel, a candidate for the autotuner (MSET_ENGINE_ALT_SHAPE):
-// smaller workgroups below 128 (at 48 a larger one); at 128 the register engine with a half-size transpose buffer
-// and a 128-register budget (two workgroups per CU instead of one; it spills about 340 registers); tiles of 16 lines
-// with 256 threads (three workgroups per CU instead of two) at 256.
+// SH = 1: the alternative shape of the batched kernel, a candidate for the autotuner (MSET_ENGINE_ALT_SHAPE): fewer threads
+// per position at 24, 32 and 64, more at 48 and 96 (the default one at 16); at 128 the register engine with a half-size
+// transpose buffer and a 128-register budget (two workgroups per CU instead of one; it spills about 340 registers); tiles
+// of 16 lines with 256 threads (three workgroups per CU instead of two) at 256.  64 and 1400 positions x 12 planes: 84 and
+// 130 us at 24 (128 threads; with 64 112 and 153), 118 and 188 at 32 (128; with 64 181 and 247); 64 and 700 at 96: 368 and
+// 1274 us (1024; with 576 486 and 1737).
 // SH = 2: launches of at most one position per CU and the one-position kernel: at 48 a workgroup of 768, at 256
 // 64-line tiles, one workgroup of 16 waves per CU with twice the default workgroup's loads in flight; the
 // default shape elsewhere.
@@ -66,12 +68,11 @@ template <> struct Cfg<64> { static constexpr int NT = 512, MINB = 4; using Eng 
 template <> struct Cfg<96> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<96, 768>; };
 template <> struct Cfg<128> { static constexpr int NT = 512, MINB = 1; using Eng = RegEngine<128>; };
 template <> struct Cfg<256> { static constexpr int NT = 512, MINB = 4; using Eng = TiledEngine<256, 512>; };
-template <> struct Cfg<16, 1> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<16, 64>; };
-template <> struct Cfg<24, 1> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<24, 64>; };
-template <> struct Cfg<32, 1> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<32, 64>; };
+template <> struct Cfg<24, 1> { static constexpr int NT = 128, MINB = 1; using Eng = LdsEngine<24, 128>; };
+template <> struct Cfg<32, 1> { static constexpr int NT = 128, MINB = 1; using Eng = LdsEngine<32, 128>; };
 template <> struct Cfg<48, 1> { static constexpr int NT = 384, MINB = 1; using Eng = LdsEngine<48, 384>; };
 template <> struct Cfg<64, 1> { static constexpr int NT = 256, MINB = 3; using Eng = LdsEngine<64, 256>; };
-template <> struct Cfg<96, 1> { static constexpr int NT = 576, MINB = 1; using Eng = LdsEngine<96, 576>; };
+template <> struct Cfg<96, 1> { static constexpr int NT = 1024, MINB = 1; using Eng = LdsEngine<96, 1024>; };
 template <> struct Cfg<128, 1> { static constexpr int NT = 512, MINB = 4; using Eng = RegEngine<128, true>; };
 template <> struct Cfg<256, 1> { static constexpr int NT = 256, MINB = 3; using Eng = TiledEngine<256, 256>; };
 template <int N> struct Cfg<N, 2> : Cfg<N> {};

@@ -84,3 +84,17 @@ def test_serving_footprint_covers_what_a_job_allocates(tmp, P, vol):
         r.snapshot()
         assert fake.fake_peak() <= serve.footprint_bytes(spec, lib.batch_slots(spec.P)), (fake.fake_peak(), serve.footprint_bytes(spec, lib.batch_slots(spec.P)))
     ''' % (vol, P))
+
+
+@pytest.mark.parametrize('n,npos,threads', [(16, 8, 64), (24, 8, 128), (32, 8, 128), (48, 8, 384), (64, 256, 512), (64, 257, 256),
+                                            (96, 8, 1024), (128, 8, 512), (256, 8, 256)])
+def test_alternative_shape(tmp, n, npos, threads):
+    fake_hip.run(tmp, '''
+        ctx = lib.Context(0)
+        upload(ctx, %d, 2, %d)
+        ctx.set_engine(lib.ENGINE_ALT_SHAPE)
+        fake.fake_reset()
+        ctx.run_batched(%d)
+        (name, _, _, threads, _), = launches('k_batch')
+        assert threads == %d, (name, threads)
+    ''' % (n, npos, npos, threads))
