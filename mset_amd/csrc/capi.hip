@@ -325,14 +325,21 @@ bool sep_fwd_lines(const mset_ctx* c) {
 }
 bool sep_grad_lines(const mset_ctx* c) { return c->n < 128 && sep_fwd_lines(c) && c->p.grad_mode == GRAD_REF; }
 constexpr int SHAPE_SEP = 3;   // its place among the workgroup shapes of a batched call
+constexpr int SHAPE_MANY = 4;  // Cfg<24, 4>
+int device_slots(mset_ctx* c, int shape);
+
+// the general routine's shape for a launch of `count` positions (multislice.hpp, Cfg<24, 4>)
+int general_shape(mset_ctx* c, int count) { return c->n == 24 && count > device_slots(c, 0) ? SHAPE_MANY : 0; }
 
 // Workgroup shape of a batched call: the alternative shape (MSET_ENGINE_ALT_SHAPE) exists for stored waves.  A
 // gradient request (fixed) stays on the general routine: the two routines' waves differ by 1e-6, which position
 // terms that cancel turn into 1e-4 of a gradient, and gradients are what callers difference.
-int shape_for(const mset_ctx* c, int waves, bool fixed) {
-    if (waves != WAVES_STORE) return 0;
-    if (c->ws->engine & MSET_ENGINE_ALT_SHAPE) return 1;
-    return sep_grad_lines(c) && !fixed ? SHAPE_SEP : 0;
+int shape_for(mset_ctx* c, int waves, bool fixed, int count) {
+    if (waves == WAVES_STORE) {
+        if (c->ws->engine & MSET_ENGINE_ALT_SHAPE) return 1;
+        if (sep_grad_lines(c) && !fixed) return SHAPE_SEP;
+    }
+    return general_shape(c, count);
 }
 
 // workgroups of the batched kernel of a workgroup shape the device keeps resident at once (1 per CU at
@@ -374,7 +381,7 @@ int batch_shape(const mset_ctx* c, int shape, bool sep, int waves, int count) {
     return c->n == 256 && sep && (waves == WAVES_STORE || waves == WAVES_CHECKPOINT) ? 2 : 0;
 }
 // the same for the forward-only kernels
-int fwd_shape(const mset_ctx* c, int count) { return c->n == 48 && count <= c->cus ? 2 : 0; }
+int fwd_shape(mset_ctx* c, int count) { return c->n == 48 && count <= c->cus ? 2 : general_shape(c, count); }
 
 // grid of a batched launch of `count` positions on S slabs: at most `want` workgroups and, when slabs take
 // several positions (count > S), a divisor of S, so that each slab's positions run on one workgroup in order
@@ -433,12 +440,13 @@ int resolve_exit_waves(mset_ctx* c, int slots, int* waves) {
     return MSET_OK;
 }
 
-int ensure_batch_buffers(mset_ctx* c, bool fixed) {
+// for launches of up to `count` positions
+int ensure_batch_buffers(mset_ctx* c, bool fixed, int count) {
     Workspace& W = *c->ws;
     int wv = WAVES_STORE;
     CHK(resolve_exit_waves(c, batch_slots(c, 0), &wv));
     W.waves = wv;
-    W.shape = shape_for(c, wv, fixed);
+    W.shape = shape_for(c, wv, fixed, count);
     const int s = batch_slots(c, W.shape);
     CHK(ensure_fixed_buffers(c, s));
     const int save_planes = wave_planes(c, wv);
@@ -536,7 +544,9 @@ int fwd_slots(const mset_ctx* c) {
 
 int issue_fwd(mset_ctx* c, float* inten) {
     const bool sep = sep_fwd(c);
-    const int grid = sep_fwd_lines(c) ? std::min(fwd_slots(c), c->npos) : batch_slots(c, 0);   // the kernels' own shape
+    const int shape = fwd_shape(c, c->npos);
+    // the grid of the kernel's own shape (the large workgroup's launch has no more positions than CUs)
+    const int grid = sep_fwd_lines(c) ? std::min(fwd_slots(c), c->npos) : batch_slots(c, shape == SHAPE_MANY ? shape : 0);
     CHK(prepare_fixed(c, grid, sep ? 1 : 0));
     PosArgs A = base_args(c);
     A.sep = sep ? 1 : 0;
@@ -545,7 +555,7 @@ int issue_fwd(mset_ctx* c, float* inten) {
     A.inten = inten;
     Timed t(c, "position_fwd");
     if (sep_fwd_lines(c)) HIPCHK(launch_sep_fwd(c->n, A, grid, false, c->stream));
-    else HIPCHK(launch_fwd(c->n, A, grid, fwd_shape(c, c->npos), c->stream));
+    else HIPCHK(launch_fwd(c->n, A, grid, shape, c->stream));
     return MSET_OK;
 }
 
@@ -553,7 +563,7 @@ int issue_fwd(mset_ctx* c, float* inten) {
 // direction, real space) and c->dpos; with apply, the steps are taken (RVol += s1 G, probe -= s2 PG,
 // positions += s3 dpos).  want: the terms to form (the gradient request forms all of them).
 int issue_grad(mset_ctx* c, int first, int count, bool apply, int want) {
-    CHK(ensure_batch_buffers(c, !apply));
+    CHK(ensure_batch_buffers(c, !apply, count));
     const bool sep = sep_batch(c);
     CHK(prepare_fixed(c, c->slots, sep ? 2 : 0));
     Workspace& W = *c->ws;
@@ -967,7 +977,7 @@ int mset_grad_noalloc(mset_ctx* c, int first, int count, float* dV, float* dprob
     auto need = [&](int S, int G) { return fixed + (size_t)S * (s_g + s_ps) + (size_t)G * (s_save + s_pl); };
     // mset_grad's slabs and grid when they fit (then the sums are bitwise mset_grad's), else as many resident
     // positions as fit, one slab each
-    const int shape = shape_for(c, WAVES_STORE, true);
+    const int shape = shape_for(c, WAVES_STORE, true, count);
     int S = std::min(grad_slabs(c, shape), count);
     int G = launch_grid(batch_slots(c, shape), count, S);
     while (G > 1 && need(S, G) > MSET_NOALLOC_SCRATCH_BYTES) G = launch_grid(G - 1, count, S);
@@ -1023,7 +1033,7 @@ int mset_waves(mset_ctx* c, int k, float* waves_out) {
     CHK(check_uploaded(c));
     if (k < 0 || k >= c->npos || !waves_out) return fail(MSET_EINVAL, "bad position index or null output");
     CHK(set_method(c, MSET_METHOD_MSET));
-    CHK(ensure_batch_buffers(c, true));
+    CHK(ensure_batch_buffers(c, true, 1));
     CHK(prepare_fixed(c, 1));
     // every plane's wave is read back: the store layout, in slot 0
     CHK(c->ws->save.ensure((size_t)(c->L + 2) * plane(c), "save waves"));
@@ -1146,10 +1156,14 @@ int mset_batch_slots(int device, int n, int* slots) {
     HIPCHK(hipGetDeviceProperties(&prop, device));
     // the routines a batched call may run: the general one (mset_grad, the exact pairing, other propagators) and, below
     // 128, the on-chip separable one (updates)
-    int per_cu = 1, per_cu_sep = 1;
+    int per_cu = 1, per_cu_alt = 1;
     HIPCHK(occupancy_batch(n, 0, &per_cu));
-    if (n < 128) HIPCHK(occupancy_sep(n, false, &per_cu_sep));
-    per_cu = std::max(per_cu, per_cu_sep);
+    if (n < 128) HIPCHK(occupancy_sep(n, false, &per_cu_alt));
+    per_cu = std::max(per_cu, per_cu_alt);
+    if (n == 24) {
+        HIPCHK(occupancy_batch(n, SHAPE_MANY, &per_cu_alt));
+        per_cu = std::max(per_cu, per_cu_alt);
+    }
     *slots = prop.multiProcessorCount * (per_cu < 1 ? 1 : per_cu);
     return MSET_OK;
 }
@@ -1342,7 +1356,8 @@ int mset_recon_error_pass(mset_recon* r, double* errs) {
     CHK(r->err_all.ensure(tot, "error-pass errors"));
     CHK(r->items.ensure(tot, "error-pass work items"));
     CHK(r->tilt_tab.ensure(T, "error-pass tilt table"));
-    int grid = std::max(1, device_slots(c0, 0));
+    const int shape = fwd_shape(c0, (int)std::min<size_t>(tot, INT_MAX));
+    int grid = std::max(1, device_slots(c0, shape == SHAPE_MANY ? shape : 0));
     if (r->ws->slot_limit > 0) grid = std::min(grid, r->ws->slot_limit);
     grid = (int)std::min<size_t>((size_t)grid, tot);
     if (plane_in_global(r->n)) CHK(r->ws->planes.ensure((size_t)grid * 2 * plane(c0), "plane buffers"));
@@ -1378,7 +1393,7 @@ int mset_recon_error_pass(mset_recon* r, double* errs) {
     {
         Timed t(c0, "position_fwd");
         if (sep_fwd_lines(c0)) HIPCHK(launch_sep_fwd(r->n, A, (int)std::min<size_t>(fwd_slots(c0), tot), true, r->stream));
-        else HIPCHK(launch_fwd_tilts(r->n, A, grid, fwd_shape(c0, (int)std::min<size_t>(tot, INT_MAX)), r->stream));
+        else HIPCHK(launch_fwd_tilts(r->n, A, grid, shape, r->stream));
     }
     std::vector<double> e(tot);
     HIPCHK(hipMemcpyAsync(e.data(), r->err_all.p, sizeof(double) * tot, hipMemcpyDeviceToHost, r->stream));

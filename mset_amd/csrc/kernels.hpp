@@ -110,9 +110,10 @@ bool position_lines_supported(int n);
 size_t position_lines_work(int n, int L);
 hipError_t launch_position_lines(int n, const PosArgs& P, int k, float2* work, hipStream_t st);
 // shape: 0 default, 1 alternative (MSET_ENGINE_ALT_SHAPE, stored waves), 2 the large workgroup for launches of
-// at most one position per CU (at 48 with stored waves; the separable 256 routine, stored or checkpointed)
+// at most one position per CU (at 48 with stored waves; the separable 256 routine, stored or checkpointed), 4 the small
+// workgroup at 24 for launches of more positions than the default shape keeps resident (any waves)
 hipError_t launch_batch(int n, const PosArgs& A, int grid, int shape, hipStream_t st);
-// shape: 0, or 2 at 48 as above
+// shape: 0, 2 at 48 or 4 at 24 as above
 hipError_t launch_fwd(int n, const PosArgs& A, int grid, int shape, hipStream_t st);
 // forward + loss over the work items A.order[0 .. A.count) of several tilts (A.tilts)
 hipError_t launch_fwd_tilts(int n, const PosArgs& A, int grid, int shape, hipStream_t st);

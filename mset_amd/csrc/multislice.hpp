@@ -59,6 +59,10 @@ namespace mset {
 // SH = 2: launches of at most one position per CU and the one-position kernel: at 48 a workgroup of 768, at 256
 // 64-line tiles, one workgroup of 16 waves per CU with twice the default workgroup's loads in flight; the
 // default shape elsewhere.
+// SH = 4: launches of more positions than the default shape keeps resident (1280), at 24: there the work of a position
+// counts and not its latency, and a workgroup of one wave leaves fewer lanes idle and more positions resident.  1400 / 2800
+// positions x 12 planes, default shape and this one: 150 / 226 and 150 / 218 us (gradient), 67 / 97 and 62 / 95 (forward),
+// 203 / 307 and 198 / 267 (checkpointed waves).
 template <int N, int SH = 0> struct Cfg;
 template <> struct Cfg<16> { static constexpr int NT = 64, MINB = 1;  using Eng = LdsEngine<16, 64>; };
 template <> struct Cfg<24> { static constexpr int NT = 192, MINB = 1; using Eng = LdsEngine<24, 192>; };
@@ -77,6 +81,7 @@ template <> struct Cfg<128, 1> { static constexpr int NT = 512, MINB = 4; using 
 template <> struct Cfg<256, 1> { static constexpr int NT = 256, MINB = 3; using Eng = TiledEngine<256, 256>; };
 template <int N> struct Cfg<N, 2> : Cfg<N> {};
 template <> struct Cfg<48, 2> { static constexpr int NT = 768, MINB = 1; using Eng = LdsEngine<48, 768>; };
+template <> struct Cfg<24, 4> { static constexpr int NT = 64, MINB = 1; using Eng = LdsEngine<24, 64>; };
 template <> struct Cfg<256, 2> { static constexpr int NT = 1024, MINB = 4; using Eng = TiledEngine<256, 1024>; };
 
 

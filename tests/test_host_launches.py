@@ -53,6 +53,7 @@ def test_batch_slots_covers_the_kernels_of_a_batched_call(tmp, n, general, separ
     fake_hip.run(tmp, '''
         n, g, s = %d, %d, %d
         fake.fake_occupancy(b'k_batch<%%d, 0' %% n, g)
+        fake.fake_occupancy(b'k_batch<%%d, 4' %% n, g)      # the small workgroup for many positions
         fake.fake_occupancy(b'k_sep_batch<%%d' %% n, s)
         slots = lib.batch_slots(n)
         per_cu = max(g, s) if n < 128 else g
@@ -98,3 +99,36 @@ def test_alternative_shape(tmp, n, npos, threads):
         (name, _, _, threads, _), = launches('k_batch')
         assert threads == %d, (name, threads)
     ''' % (n, npos, npos, threads))
+
+
+def test_many_positions_at_24_take_the_small_workgroup(tmp):
+    """one position more than the default shape keeps resident; the grid is that of the shape that is launched"""
+    fake_hip.run(tmp, '''
+        fake.fake_occupancy(b'k_batch<24, 0', 3)
+        fake.fake_occupancy(b'k_batch<24, 4', 7)
+        for npos, shape, threads in ((3 * 256, 0, 192), (3 * 256 + 1, 4, 64)):
+            ctx = lib.Context(0)
+            upload(ctx, 24, 2, npos, separable=False)
+            for wv in (lib.EXIT_WAVES_STORE, lib.EXIT_WAVES_CHECKPOINT):
+                ctx.set_exit_waves(wv)
+                fake.fake_reset()
+                ctx.run_batched(npos)
+                ctx.grad()
+                for name, gx, _, nt, _ in launches('k_batch<'):
+                    assert 'k_batch<24, %%d' %% shape in name and nt == threads and gx == npos, (name, gx, nt)
+            fake.fake_reset()
+            ctx.error_resident()
+            (name, gx, _, nt, _), = launches('k_fwd<')
+            assert 'k_fwd<24, %%d' %% shape in name and nt == threads and gx == npos, (name, gx, nt)
+            ctx.run_batched(700)                     # the launches of a pass decide, not the positions of the tilt
+            fake.fake_reset()
+            ctx.run_batched(700)
+            assert all(nt == 192 for _, _, _, nt, _ in launches('k_batch<'))
+            ctx.close()
+        r = recon(24, 16, (500, 600), angles=(0., 10.))
+        r.set_engine(lib.ENGINE_GENERAL)
+        fake.fake_reset()
+        r.error_pass()
+        (name, gx, _, nt, _), = launches('k_fwd<')
+        assert 'k_fwd<24, 4' in name and nt == 64 and gx == 1100, (name, gx, nt)
+    '''.replace('%%', '%'))
