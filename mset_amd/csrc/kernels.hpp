@@ -126,7 +126,7 @@ hipError_t launch_plane_fft(int n, const float2* in, float2* out, const float2* 
 bool plane_in_global(int n);     // the position kernels keep the plane in global memory (planes buffer)
 hipError_t occupancy_batch(int n, int shape, int* blocks_per_cu);
 // on-chip separable routine (sep_lines.hip): A.pfac, the multislice operator; forward-only up to 128, below it the
-// gradient kernels with the reference pairing and stored waves.  launch_sep_plain: as launch_plain.
+// gradient kernels with the reference pairing and stored waves.  launch_sep_plain: as launch_plain, up to 64.
 hipError_t launch_sep_batch(int n, const PosArgs& A, int grid, hipStream_t st);
 hipError_t launch_sep_plain(int n, const PosArgs& A, int k, hipStream_t st);
 hipError_t launch_sep_fwd(int n, const PosArgs& A, int grid, bool tilts, hipStream_t st);

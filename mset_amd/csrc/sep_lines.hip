@@ -3,15 +3,25 @@
 
 namespace mset {
 
-#define MSET_SEP_DISPATCH(N, BODY)                           \
-    switch (N) {                                             \
-        case 16: { constexpr int NN = 16; BODY; } break;     \
-        case 24: { constexpr int NN = 24; BODY; } break;     \
-        case 32: { constexpr int NN = 32; BODY; } break;     \
-        case 48: { constexpr int NN = 48; BODY; } break;     \
-        case 64: { constexpr int NN = 64; BODY; } break;     \
-        case 96: { constexpr int NN = 96; BODY; } break;     \
-        default: return hipErrorInvalidValue;                \
+#define MSET_SEP_CASES_64(...)                               \
+    case 16: { constexpr int NN = 16; __VA_ARGS__; } break;  \
+    case 24: { constexpr int NN = 24; __VA_ARGS__; } break;  \
+    case 32: { constexpr int NN = 32; __VA_ARGS__; } break;  \
+    case 48: { constexpr int NN = 48; __VA_ARGS__; } break;  \
+    case 64: { constexpr int NN = 64; __VA_ARGS__; } break;
+
+#define MSET_SEP_DISPATCH(N, ...)                               \
+    switch (N) {                                                \
+        MSET_SEP_CASES_64(__VA_ARGS__)                          \
+        case 96: { constexpr int NN = 96; __VA_ARGS__; } break; \
+        default: return hipErrorInvalidValue;                   \
+    }
+
+// sizes whose sequential path is a launch per position (from 96 on it is a chain of line passes)
+#define MSET_SEP_DISPATCH_64(N, ...)          \
+    switch (N) {                              \
+        MSET_SEP_CASES_64(__VA_ARGS__)        \
+        default: return hipErrorInvalidValue; \
     }
 
 hipError_t launch_sep_batch(int n, const PosArgs& A, int grid, hipStream_t st) {
@@ -22,7 +32,7 @@ hipError_t launch_sep_batch(int n, const PosArgs& A, int grid, hipStream_t st) {
 
 hipError_t launch_sep_plain(int n, const PosArgs& A, int k, hipStream_t st) {
     if (!A.pfac || A.sset || A.grad_mode != GRAD_REF) return hipErrorInvalidValue;
-    MSET_SEP_DISPATCH(n, hipLaunchKernelGGL((k_sep_plain<NN>), dim3(1), dim3(SepCfg<NN>::NT), 0, st, A, k))
+    MSET_SEP_DISPATCH_64(n, hipLaunchKernelGGL((k_sep_plain<NN>), dim3(1), dim3(SepCfg<NN>::NT), 0, st, A, k))
     return hipGetLastError();
 }
 

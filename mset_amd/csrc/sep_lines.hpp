@@ -1,5 +1,5 @@
 // sep_lines.hpp -- the separable position routine with the plane on chip (CDNA4, gfx950): forward-only up to
-// N = 128, gradients and the one-position kernel below.
+// N = 128, gradients below, the one-position kernel up to 64.
 //
 // A separable propagator p(kx, ky) = px(kx) py(ky) makes a propagation step two half-steps along one axis
 // each, which commute; alternating their order from plane to plane (see process_sep in multislice.hpp) leaves
@@ -430,7 +430,7 @@ template <int N> __global__ __launch_bounds__((SepCfg<N>::NT), (SepCfg<N>::MINB)
 }
 
 template <int N> __global__ __launch_bounds__((SepCfg<N>::NT), (SepCfg<N>::MINB)) void k_sep_plain(PosArgs A, int k) {
-    MSET_SEP_LDS(N, (N <= 64 ? 2 : 1))
+    MSET_SEP_LDS(N, 2)
     position_sep_lines<N, K_PLAIN>(A, k, 0, 0, true, E, phx, phy, px, py, red);
 }
 

@@ -45,6 +45,12 @@ void fake_reset() {
     g_peak = g_bytes;
 }
 const char* fake_log() { return g_log.c_str(); }
+const char* fake_kernels() {                              // every kernel of the library, one a line
+    static std::string all;
+    all.clear();
+    for (const auto& kv : g_names) all += kv.second + "\n";
+    return all.c_str();
+}
 int fake_captures() { return g_captures; }
 int fake_replays() { return g_replays; }
 int fake_stale_replays() { return g_stale_replays; }

@@ -11,7 +11,7 @@ PRELUDE = '''
 import ctypes as C
 import sys
 fake = C.CDLL(%(so)r, mode=C.RTLD_GLOBAL)
-fake.fake_log.restype = C.c_char_p
+fake.fake_log.restype = fake.fake_kernels.restype = C.c_char_p
 fake.fake_bytes.restype = fake.fake_peak.restype = C.c_size_t
 fake.fake_fail_malloc.argtypes = fake.fake_device_memory.argtypes = [C.c_size_t]
 fake.fake_occupancy.argtypes = [C.c_char_p, C.c_int]

@@ -132,3 +132,19 @@ def test_many_positions_at_24_take_the_small_workgroup(tmp):
         (name, gx, _, nt, _), = launches('k_fwd<')
         assert 'k_fwd<24, 4' in name and nt == 64 and gx == 1100, (name, gx, nt)
     '''.replace('%%', '%'))
+
+
+def test_sequential_kernels_are_the_ones_that_are_reached(tmp):
+    """the one-position separable kernel is built where the sequential path launches it, and nowhere else"""
+    fake_hip.run(tmp, '''
+        ctx = lib.Context(0)
+        reached = set()
+        for n in (16, 24, 32, 48, 64, 96, 128, 256):
+            upload(ctx, n, 3, 2)
+            fake.fake_reset()
+            ctx.run_resident()
+            reached |= {name for name, *_ in launches('k_sep_plain')}
+            assert bool(launches('k_line_pass')) == (n >= 96)
+        built = {l for l in fake.fake_kernels().decode().splitlines() if 'k_sep_plain' in l}
+        assert built == reached and len(built) == 5, built ^ reached
+    ''')
