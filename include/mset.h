@@ -215,8 +215,10 @@ int mset_recon_set_tilt(mset_recon* r, int j, const double* angles, const float*
                         int num_scan_pos, const float* xlist, const float* ylist, const float* measured);
 int mset_recon_set_steps(mset_recon* r, const float* steps);
 /* One update pass.  batch: positions per mini-batch (MSET_PATH_BATCHED).  use_graph: capture the pass in
- * a hipGraph on first use and replay it afterwards.  error_out (nullable): mean over tilts of the
- * update-pass errors. */
+ * a hipGraph on first use and replay it afterwards; the results are those of the eager pass.  A captured pass holds a
+ * node per kernel launch, and a sequential pass is 3 launches per position, or with a separable propagator from 96 x 96
+ * up 2 L + 6: one of more than 65536 launches is issued eagerly (replayed, it would not be faster), and so is every pass
+ * while profiling is on.  error_out (nullable): mean over tilts of the update-pass errors. */
 int mset_recon_iterate(mset_recon* r, int path, int batch, int use_graph, int positivity, double* error_out);
 /* Error pass (Run_MSET_recon.m:189-239): errs[j] for every tilt at the current rec. */
 int mset_recon_error_pass(mset_recon* r, double* errs);

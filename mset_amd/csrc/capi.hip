@@ -816,7 +816,7 @@ int check_recon(mset_recon* r) {
 
 // A sequential pass in more launches than this is issued eagerly even when a graph is asked for: a captured
 // pass has a node per launch, and the host issues the launches faster than they run (3 tilts of 64 positions at
-// 128 x 128, 3.5k launches: 16.6 ms eager, 16.5 ms replayed).
+// 128 x 128 x 16 planes, 7.3k launches: 32.8 ms eager, 32.7 ms replayed, 10 ms for the capture).
 constexpr size_t PLAIN_GRAPH_LAUNCHES = 65536;
 
 size_t plain_launches(const mset_recon* r) {

@@ -403,6 +403,8 @@ class Recon:
         _chk(self._L.mset_recon_set_steps(self._h, _ptr(s)))
 
     def iterate(self, path=PATH_BATCHED, batch=256, use_graph=False, positivity=True, want_error=True):
+        """one update pass; use_graph replays it from a captured graph (a sequential pass of more than 65536 launches
+        is issued eagerly all the same)"""
         e = np.zeros(1, np.float64)
         _chk(self._L.mset_recon_iterate(self._h, int(path), int(batch), int(bool(use_graph)), int(bool(positivity)),
                                         _ptr(e) if want_error else None))

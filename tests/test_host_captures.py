@@ -54,3 +54,42 @@ def test_passes_that_grow_nothing_keep_the_capture(tmp):
         r.iterate(lib.PATH_BATCHED, 4, use_graph=True)
         assert fake.fake_captures() == n
     ''')
+
+
+# 3 launches per position below 96 x 96, 2 L + 6 from there on
+@pytest.mark.parametrize('n,nz,limit', [(16, 16, 65536 // 3), (96, 256, 65536 // 518)])
+def test_long_sequential_passes_are_issued_eagerly(tmp, n, nz, limit):
+    """a graph is asked for on both sides of the limit; the launches of a pass are the same"""
+    fake_hip.run(tmp, '''
+        n, nz, limit = %d, %d, %d
+        counts = []
+        for npos in (limit, limit + 1):
+            r = recon(n, nz, npos, angles=(0.,))
+            fake.fake_reset()
+            r.iterate(lib.PATH_PLAIN, 1, use_graph=True)
+            first = [row[:4] for row in launches() if not row[4]]
+            counts.append(len([row for row in first if 'position' in row[0] or 'plain' in row[0] or 'line_pass' in row[0]
+                               or 'trans' in row[0]]))
+            assert fake.fake_captures() == (npos == limit), npos
+            fake.fake_reset()
+            r.iterate(lib.PATH_PLAIN, 1, use_graph=True)
+            assert fake.fake_replays() == (npos == limit)
+            if npos > limit:
+                assert [row[:4] for row in launches()] == first
+            r.close()
+        assert 0.6 * 65536 < counts[0] <= 65536, counts        # the estimate is at least the launches
+    ''' % (n, nz, limit))
+
+
+def test_profiled_passes_are_issued_eagerly(tmp):
+    fake_hip.run(tmp, '''
+        r = recon(64, 16, 4)
+        r.iterate(lib.PATH_BATCHED, 4, use_graph=True)
+        r.profile(True)
+        r.iterate(lib.PATH_BATCHED, 4, use_graph=True)
+        assert (fake.fake_captures(), fake.fake_replays()) == (1, 0)
+        assert r.profile_read('position_batch')[0] == 2
+        r.profile(False)
+        r.iterate(lib.PATH_BATCHED, 4, use_graph=True)
+        assert (fake.fake_captures(), fake.fake_replays()) == (2, 0)
+    ''')
