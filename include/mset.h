@@ -150,14 +150,23 @@ int mset_exit_waves(mset_ctx* ctx, int* resolved, size_t* bytes_per_slot);
  * no counterpart in the reference: fewer slots hold less scratch and may keep more of it in cache. */
 int mset_set_slot_limit(mset_ctx* ctx, int slots);
 /* Engine flags of the position kernels, a tuning knob with no counterpart in the reference; every choice
- * agrees with the FP64 oracle to the same tolerances.  AUTO (0, the default): at 256 x 256, when the
- * propagator factors as p(kx, ky) = px(kx) py(ky) (the Fresnel propagator of Func_generate_propagator.m
- * does, checked at upload), the forward kernels and the reference-pairing batched gradient with stored
- * waves run the separable routine, which applies the two 1D half-steps of neighbouring planes in one pass
- * over the plane (half the passes).  GENERAL: always the 2D routine.  ALT_SHAPE: the batched kernel with
- * stored waves runs the alternative workgroup shape of its plane size: fewer threads per position of the LDS
- * engine at 24, 32, 64 and 96 (more at 48, as many at 16), at 128 the register engine with a half-size transpose
- * buffer and a 128-register budget (two workgroups per CU instead of one), at 256 16-line tiles with 256
+ * agrees with the FP64 oracle to the same tolerances.
+ * AUTO (0, the default): when the propagator factors as p(kx, ky) = px(kx) py(ky) (the Fresnel propagator of
+ * Func_generate_propagator.m does, checked at upload), the multislice operator runs separable routines, which
+ * apply the two 1D half-steps of neighbouring planes in one pass over the plane (half the passes):
+ *   - error and simulation calls, at every size;
+ *   - sequential updates with the reference pairing, at every size;
+ *   - mini-batch updates with the reference pairing, below 128 with stored waves, at 256 with stored or checkpointed
+ *     ones;
+ *   - mset_grad (the same waves) and mset_grad_noalloc with the reference pairing, at 256.
+ * The general routine, which transforms along both axes for every step, runs the rest.  So below 128 a mini-batch
+ * update and mset_grad at the same state come from different routines: they agree to FP32 rounding (within 1e-5 of
+ * each gradient term's norm), not bit for bit, and where a position's terms cancel, to that error of what cancels.
+ * GENERAL: always the general routine, for every call.
+ * ALT_SHAPE: batched calls with stored waves run the alternative workgroup shape of their plane size.  Below 256 that
+ * is a shape of the general routine: 128 threads per position at 24 and 32, 384 at 48, 256 at 64 (from two positions
+ * per CU on), 1024 at 96, the default 64 at 16; at 128 the register engine with a half-size transpose buffer and a
+ * 128-register budget (two workgroups per CU instead of one).  At 256, of the routine that runs: 16-line tiles with 256
  * threads (three workgroups per CU instead of two).  The flags combine. */
 #define MSET_ENGINE_AUTO 0
 #define MSET_ENGINE_GENERAL 1

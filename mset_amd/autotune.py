@@ -1,7 +1,7 @@
 """Autotuner of the batched path: picks the engine, the persistent grid and the mini-batch size by timing
 them on the workload itself.
 
-Tunables (both leave the kernels' arithmetic unchanged):
+Tunables:
   slots  the persistent grid of the batched kernels (mset_set_slot_limit; 0 = every resident workgroup).
          Fewer resident positions hold less scratch (saved waves and, at 256 x 256, the plane buffers) and
          keep more of it in L2 / MALL; more of them hide memory latency better.  Gradient slabs are
@@ -10,12 +10,12 @@ Tunables (both leave the kernels' arithmetic unchanged):
   batch  positions per launch of an update pass (the mini-batch size), from the range the caller
          allows: it sets how many launches, reductions and updates a pass makes and how well the last
          wave of workgroups fills the device.
-  engine mset_set_engine flags: the plane routine at 256 x 256 (the separable-propagator routine, one pass
+  engine mset_set_engine flags.  At 256 x 256: the plane routine (the separable-propagator routine, one pass
          over the plane per propagation step, or the general 2D routine, two passes per step) and the
-         workgroup shape of the batched kernel at every size (the default shape, or the alternative one:
-         fewer threads per position of the LDS engine (more at 48), two register-engine workgroups per CU
-         at 128, 16- instead of 32-line tiles at 256).  Engines sum in different orders: results agree to FP32
-         rounding.
+         workgroup shape (32- or 16-line tiles).  Below it the default, against the general routine in its
+         alternative shape: with a separable propagator and the reference pairing that is another routine
+         below 128, else only another number of threads per position (at 128 two register-engine workgroups
+         per CU).  Engines sum in different orders: results agree to FP32 rounding.
 
 Each candidate runs one update pass from a snapshot of the tilt series, which is restored afterwards,
 so tuning leaves the reconstruction unchanged.  The kernels are timed with HIP events on the series'
@@ -44,15 +44,15 @@ def slot_candidates(n, fracs=(1.0, 0.5, 0.25), device=0):
 
 
 def engine_candidates(n):
-    """Engines worth timing at plane size n: the default and the alternative workgroup shape, and at 256 the
-    general routine (the separable one is the default)."""
+    """Engines worth timing at plane size n: the default and the alternative workgroup shape (below 256 one of the
+    general routine), and at 256 the general routine in its default shape (the separable one is the default)."""
     if n == 256:
         return (lib.ENGINE_AUTO, lib.ENGINE_ALT_SHAPE, lib.ENGINE_GENERAL)
     return (lib.ENGINE_AUTO, lib.ENGINE_ALT_SHAPE)
 
 
 def engine_name(e):
-    """readable name of mset_set_engine flags"""
+    """readable name of mset_set_engine flags (the alternative shape below 256 is one of the general routine)"""
     parts = ['general routine' if e & lib.ENGINE_GENERAL else 'default routine',
              'alternative shape' if e & lib.ENGINE_ALT_SHAPE else 'default shape']
     return ', '.join(parts)

@@ -314,7 +314,8 @@ class Context:
         _chk(self._L.mset_set_slot_limit(self._h, int(slots)))
 
     def set_engine(self, engine):
-        """ENGINE_AUTO (separable routine at 256 when the propagator factors) or ENGINE_GENERAL"""
+        """ENGINE_AUTO (separable routines where the propagator factors), or ENGINE_GENERAL and ENGINE_ALT_SHAPE,
+        which combine (mset_set_engine)"""
         _chk(self._L.mset_set_engine(self._h, int(engine)))
 
     def exit_waves(self):
@@ -441,7 +442,7 @@ class Recon:
         _chk(self._L.mset_recon_set_slot_limit(self._h, int(slots)))
 
     def set_engine(self, engine):
-        """ENGINE_AUTO or ENGINE_GENERAL for the series' passes"""
+        """the same for the series' passes (mset_recon_set_engine)"""
         _chk(self._L.mset_recon_set_engine(self._h, int(engine)))
 
     def snapshot(self):
