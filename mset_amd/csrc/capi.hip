@@ -116,7 +116,9 @@ struct Workspace {
     }
 };
 
-thread_local std::weak_ptr<Workspace> g_call_ws;   // set by the checks that every entry point begins with
+// Set by the checks that the entry points begin with, none in a call that creates one: a workspace other than the call's
+// own may be in use on another thread.
+thread_local std::weak_ptr<Workspace> g_call_ws;
 
 bool give_back_kept() {
     const std::shared_ptr<Workspace> W = g_call_ws.lock();
@@ -1235,6 +1237,7 @@ int mset_recon_create(mset_recon** out, int device, const mset_params* common, i
     r->ws = std::make_shared<Workspace>();
     r->prof = std::make_shared<ProfMap>();
     const size_t nv = (size_t)r->n * r->n * r->nz;
+    g_call_ws.reset();
     CHK(r->rec.ensure(nv, "reconstruction"));
     HIPCHK(hipMemcpyAsync(r->rec.p, rec, sizeof(float) * nv, hipMemcpyHostToDevice, r->stream));
     HIPCHK(hipStreamSynchronize(r->stream));

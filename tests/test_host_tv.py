@@ -76,3 +76,24 @@ def test_allocations_that_never_fit_are_refused_and_leave_the_context_usable(tmp
         ctx.run_batched(4)
         ctx.tv(np.ones((24, 64, 64), np.float32), 0.5, 1)
     ''')
+
+
+@pytest.mark.parametrize('what', ['recon', 'context'])
+def test_scratch_of_another_context_is_left_alone(tmp, what):
+    """it may be in use on another thread: what this thread called last says nothing about it"""
+    fake_hip.run(tmp, '''
+        a = lib.Context(0)
+        b = lib.Context(0)
+        a.tv(np.ones((24, 64, 64), np.float32), 0.5, 1)
+        kept = fake.fake_bytes()
+        fake.fake_device_memory(kept + 1000)
+        try:
+            if %r == 'recon':
+                recon(64, 16, 4)
+            else:
+                upload(b, 64, 24, 4)
+            raise SystemExit('fitted')
+        except lib.MsetError as e:
+            assert e.code == lib.MSET_ENOMEM
+        assert fake.fake_bytes() >= kept, (fake.fake_bytes(), kept)
+    ''' % what)
